@@ -1,42 +1,54 @@
 // mx_edge_fused.hip -- fused 3-D MakeEdgeScal: PPM, predictor, transverse
 // and edge states of one scalar in a single z-marching kernel.
 //
-// A block owns a 32 x 8 tile of cell columns of one box, grown by one cell in
-// x and y (34 x 10 columns, one thread each), and marches up a chunk [z0, z1]
-// of the box's planes, one cell plane q per step (plus q = z0 - 1 and
-// q = z1 + 1, whose states the chunk's first and last faces need).
+// A block owns a tile of cell columns of one box (16 x 11 by default), grown
+// by one cell in x and y (18 x 13 columns, one thread each), and marches up a
+// chunk [z0, z1] of the box's planes, one cell plane q per step (plus
+// q = z0 - 1 and q = z1 + 1, whose states the chunk's first and last faces
+// need).
 //
 // The reference formulas (MaestroMakeEdgeScalars.cpp: Predictor :662-863,
-// Transverse :865-1359, Edges :1361-1667; MaestroPPM.cpp) are regrouped, not
-// changed:
+// Transverse :865-1359, Edges :1361-1667; MaestroPPM.cpp) are evaluated upwind
+// first:
+//   * a face's predictor, corner-coupled and edge states are selected by the
+//     sign of the face velocity, so a face evaluates the PPM limiter, the
+//     trace, the transverse and the edge corrections of its upwind cell only
+//     (the cell's LDS slot is the face's own or its low neighbour's).  The
+//     reference forms both sides and selects; the selected value is the same
+//     expression with the same operands in the same order;
+//   * a face with |u| <= rel_eps averages both sides.  Its two states are the
+//     plain cell values (the trace is off), so the rare path re-reads them;
+//   * domain sides: an extrapolating or even side takes the inside cell's
+//     state, ext_dir the outside value, an odd side zero, at every stage, so a
+//     side fixes the face's upwind cell or its value;
 //   * a PPM face value (type 1: the limited 4th-order interpolant; type 2: the
-//     Colella-Sekora face value) is computed once per face and read by both
-//     cells beside it; sigma = |u| dt / dx likewise, once per face;
-//   * each transverse correction of a corner-coupled state,
-//     dt/6h (u_T(+) + u_T(-)) (simh_T(+) - simh_T(-)), depends only on the cell
-//     it is taken across, so it is computed once per cell and direction T and
-//     used by every face state that crosses that cell (the left state of the
-//     face above it and the right state of the face below); the edge-state
-//     corrections likewise;
-//   * every such term is evaluated by the reference's expression in the
-//     reference's operand order, and subtracted in the reference's order, so
-//     all results are bit-identical to the per-point form.
+//     Colella-Sekora face value) is computed once per face and read by the
+//     faces whose upwind cell it bounds.
 // PPM boundary stencils (ext_dir / hoextrap within two or three cells of the
 // domain edge) fall back to the full per-cell routine of mx_device.H.
 //
-// Per step q a block runs seven phases separated by barriers:
-//   A  stage plane q of s, the x- and y-MAC velocities and their sigma in LDS;
-//      shift the column's z window (s, w, force) in registers;
-//   B1 PPM face values of plane q (x, y) into LDS; PPM of cell q in z
-//      (register window) and the upwind state simhz on z-face q;
-//   B2 PPM of plane q in x and y (cell limiter + trace);
-//   C  predictor states and upwind states simhx, simhy of plane q;
-//   D1 per-cell transverse terms: x, y of plane q, z of plane q-1;
-//   D2 corner-coupled states simhxy, simhyx (plane q), simhxz, simhyz (plane
-//      q-1), simhzx, simhzy (z-face q, in registers);
-//   E1 per-cell edge terms of plane q-1 (LDS) and of plane q (registers);
-//   E2 edge states of plane q-1 (x and y faces) and of z-face q.
+// Per step q a block runs three phases separated by barriers:
+//   1  the edge states of step q - 1 (x and y faces of plane q - 2, z-face
+//      q - 1); the PPM face values of plane q;
+//   2  limiter, trace and upwind state of the x, y and z faces of cell q; the z
+//      transverse term of plane q - 1;
+//   3  corner-coupled states simhxy, simhyx (plane q), simhxz, simhyz (plane
+//      q - 1), simhzx, simhzy (z-face q, in registers) and the z edge terms;
+//      plane q + 1 (loaded into registers since phase 1) goes to LDS.
+// A phase is straight-line code: every thread evaluates it, columns past the
+// tile on clamped loads and neighbouring LDS slots, and only stores and the rare
+// paths are predicated.
+//
+// What bounds it: VALU issue and the latency of the dependent FP64 chains
+// between barriers, not HBM (3.5 + 2.6 GB move per 256^3 launch of 5 scalars).
+// One wave alone takes 10.7 thousand cycles a step for 510 VALU instructions,
+// so waves in flight decide: the advective ppm_type 1 kernel is held to 128
+// VGPRs and 40 KB of LDS, 4 blocks a CU (3.11 ms at 3 blocks, 2.68 ms at 4).
+// Measured per 256^3 launch against evaluating both sides of every face in
+// seven phases: ppm_type 1 2.68 ms (3.74), VALU 65% busy (55%); ppm_type 2
+// 4.51 ms (5.48); conservative, 128^3 and 3 species, 0.38 ms (0.46).
 #include <algorithm>
+#include <climits>
 
 #include "mx_internal.H"
 
@@ -54,22 +66,32 @@ __host__ __device__ constexpr int fused_nt(int tx, int ty) {
     return ((tx + 2) * (ty + 2) + 63) / 64 * 64;
 }
 
+// the register budget, as waves per SIMD: 4 (128 VGPRs) where the advective
+// ppm_type 1 kernel fits it and 4 blocks' LDS fit a CU, else 3 (168)
+constexpr int fused_wpe(int ppm, bool cons, int tx, int ty, int mode) {
+    return ppm == 1 && !cons && mode == 0 && tx * ty == 16 * 11 ? 4 : 3;
+}
+
 struct FBox {
-    int lo[3], hi[3];
+    int hi[3];
     DA s, fo;
     DA um[3], se[3];
-    // geometry of the box's level
-    double dx[3];
+    // plane strides in bytes: s, force, umac x / y / z, sedge x / y / z
+    long long ks[8];
+    // the box's level: its domain and, per direction, the cell width
     int domlo[3], domhi[3];
+    DivBy h[3];
     // the flux epilogue (FComp::flux): the fluxes and the level's base
     // state at cell heights (bc_a, bc_b: old, new) and at edges (be_a, be_b)
     DA sf[3];
     const double *bc_a, *bc_b, *be_a, *be_b;
 };
 
-// one block's work: a tile of one box, chunk tzc of its planes
+// one block's work: nx x ny columns and nz planes of one box from (x0, y0, z0)
 struct FTile {
-    int box, tx, ty, tzc;
+    int box, x0, y0, z0;
+    int nx, ny, nz;
+    int zgen;  // bits: a z side (0 low, 1 high) in reach needs more than the upwind cell
 };
 
 struct FComp {
@@ -82,691 +104,734 @@ struct FComp {
 };
 
 struct FArgs {
-    int start_scomp;
+    double dt, rel_eps, dt2, dt3, tf, ef;  // tf, ef: h x the factors of the
+                                           // transverse and edge terms
     int num_comp;
     int is_vel;
-    int tz;  // planes per chunk
 };
+
+typedef __attribute__((address_space(1))) const char gcc;
+typedef __attribute__((address_space(1))) char gc;
+
+// a double at a uniform base plus a 32-bit byte offset.  The empty asm keeps
+// the offset's widening beside the access, where the compiler folds it into
+// the addressing mode (one VGPR per address, no 64-bit add).
+__device__ __forceinline__ double gload(gcc* base, unsigned off) {
+    asm("" : "+v"(off));
+    return *(gcd*)(base + off);
+}
+__device__ __forceinline__ void gstore(gc* base, unsigned off, double v) {
+    asm("" : "+v"(off));
+    *(gd*)(base + off) = v;
+}
+
+// The table's pointer, behind the optimiser's back: what is read from it is
+// read (by scalar loads, from the constant address space) where it is used, not
+// kept in scalar registers over the whole loop (which overflow into vector
+// lanes, two vector instructions per use).
+typedef __attribute__((address_space(4))) const FBox cbox;
+__device__ __forceinline__ cbox* fresh(const FBox* p) {
+    unsigned long long a = (unsigned long long)p;
+    asm("" : "+s"(a));
+    return (cbox*)a;
+}
 
 // the flux of edge state `se` on d-face (i, j, k) (MakeRhoHFlux, planar,
 // MaestroMakeFlux.cpp:557-620: umac (rhoh0_edge + sedge), the base state at
 // the face's height, averaged over old and new, from the edge-centred state on
 // vertical faces)
 __device__ __forceinline__ void flux_store(const FBox& B, int d, int i, int j, int k, int comp,
-                                           int kind, double um, double se, bool vertical) {
+                                           int kind, double um, double se) {
     double f;
     if (kind == 1) {
-        const double b0 = vertical ? 0.5 * (B.be_a[k] + B.be_b[k]) : 0.5 * (B.bc_a[k] + B.bc_b[k]);
-        f = um * (b0 + se);
+        gcd* a = (gcd*)(d == 2 ? B.be_a : B.bc_a);
+        gcd* b = (gcd*)(d == 2 ? B.be_b : B.bc_b);
+        f = um * (0.5 * (a[k] + b[k]) + se);
     } else {
         f = um * se;
     }
-    B.sf[d](i, j, k, comp) = f;
+    ((gd*)B.sf[d].p)[B.sf[d].off(i, j, k, comp)] = f;
 }
 
-// predictor-style boundary overrides on a (left, right) pair at face `pos`
-__device__ __forceinline__ void bc_pair(int pos, int dlo, int dhi, int bclo, int bchi,
-                                        bool vel_normal, double sL, double sR, double& l,
-                                        double& r) {
-    if (pos == dlo) {
-        if (bclo == MX_BC_EXT_DIR) {
-            l = sL;
-            r = l;
-        } else if (bclo == MX_BC_FOEXTRAP || bclo == MX_BC_HOEXTRAP) {
-            if (vel_normal) r = dmin(r, 0.0);
-            l = r;
-        } else if (bclo == MX_BC_REFLECT_EVEN) {
-            l = r;
-        } else if (bclo == MX_BC_REFLECT_ODD) {
-            l = 0.0;
-            r = 0.0;
-        }
-    } else if (pos == dhi + 1) {
-        if (bchi == MX_BC_EXT_DIR) {
-            l = sR;
-            r = l;
-        } else if (bchi == MX_BC_FOEXTRAP || bchi == MX_BC_HOEXTRAP) {
-            if (vel_normal) l = dmax(l, 0.0);
-            r = l;
-        } else if (bchi == MX_BC_REFLECT_EVEN) {
-            r = l;
-        } else if (bchi == MX_BC_REFLECT_ODD) {
-            l = 0.0;
-            r = 0.0;
-        }
+// What an acting boundary condition makes of the face on a domain side
+// (MaestroMakeEdgeScalars.cpp:709-738, 931-961, 1446-1480): foextrap, hoextrap
+// and reflect_even take the inside cell's state at every stage, ext_dir the
+// outside cell's value, reflect_odd zero.
+enum { kInside = 1, kOutside = 2, kZero = 3 };
+__device__ __forceinline__ int side_kind(int bc) {
+    if (bc == MX_BC_EXT_DIR) return kOutside;
+    if (bc == MX_BC_REFLECT_ODD) return kZero;
+    return bc == MX_BC_FOEXTRAP || bc == MX_BC_HOEXTRAP || bc == MX_BC_REFLECT_EVEN ? kInside : 0;
+}
+
+// one direction's domain sides as the faces at `pos` see them
+struct Side {
+    bool lo, hi;  // on an acting low / high side: the upwind cell is the inside one
+    bool fixed;   // its value is not computed (ext_dir, reflect_odd)
+    bool zero;    // reflect_odd
+    bool clamp;   // the normal velocity does not enter through it
+    __device__ __forceinline__ Side(int pos, int dlo, int dhi, int bclo, int bchi, bool normal) {
+        const int kl = side_kind(bclo), kh = side_kind(bchi);
+        lo = kl && pos == dlo;
+        hi = kh && pos == dhi + 1;
+        const int k = lo ? kl : (hi ? kh : 0);
+        const int bc = lo ? bclo : bchi;
+        fixed = k >= kOutside;
+        zero = k == kZero;
+        clamp = normal && k == kInside && bc != MX_BC_REFLECT_EVEN;
     }
-}
-
-__device__ __forceinline__ double upwind(double l, double r, double u, double thr) {
-    double res = (u > 0.0) ? l : r;
-    res = (dabs(u) > thr) ? res : 0.5 * (l + r);
-    return res;
-}
-
-// final edge-state override (MaestroMakeEdgeScalars.cpp:1450-1480)
-__device__ __forceinline__ double bc_edge(double res, int pos, int dlo, int dhi, int bclo,
-                                          int bchi, bool vel_normal, double sL, double sR,
-                                          double sedgel, double sedger) {
-    if (pos == dlo) {
-        if (bclo == MX_BC_EXT_DIR) {
-            res = sL;
-        } else if (bclo == MX_BC_FOEXTRAP || bclo == MX_BC_HOEXTRAP) {
-            res = vel_normal ? dmin(sedger, 0.0) : sedger;
-        } else if (bclo == MX_BC_REFLECT_EVEN) {
-            res = sedger;
-        } else if (bclo == MX_BC_REFLECT_ODD) {
-            res = 0.0;
-        }
-    } else if (pos == dhi + 1) {
-        if (bchi == MX_BC_EXT_DIR) {
-            res = sR;
-        } else if (bchi == MX_BC_FOEXTRAP || bchi == MX_BC_HOEXTRAP) {
-            res = vel_normal ? dmax(sedgel, 0.0) : sedgel;
-        } else if (bchi == MX_BC_REFLECT_EVEN) {
-            res = sedgel;
-        } else if (bchi == MX_BC_REFLECT_ODD) {
-            res = 0.0;
-        }
+    // a stage's state x, s being the predictor's state (final on a fixed side)
+    __device__ __forceinline__ double set(double x, double s) const {
+        if (clamp) x = lo ? dmin(x, 0.0) : dmax(x, 0.0);
+        return fixed ? s : x;
     }
-    return res;
+};
+
+// a face's upwind choice: `left` its low cell, `both` the average (|u| <=
+// rel_eps); `traced`: the cell's state is traced to it (ppm_trace: u > rel_eps
+// from the left, u < -rel_eps from the right)
+struct Face {
+    bool left, both, traced;
+    __device__ __forceinline__ Face(double u, double eps, bool lo, bool hi) {
+        const bool up = u > 0.0, off = dabs(u) > eps;
+        left = (up | hi) & !lo;
+        both = !(off | lo | hi);
+        traced = off & !(left ^ up);
+    }
+};
+
+// trace of the upwind cell to its face (ppm_trace of mx_device.H for one
+// side): A the edge value at the face, B the cell's other edge value.
+// sp - h (sp - sm - c s6) and sm + h (sp - sm + c s6) are both
+// A + h ((B - A) + c s6).
+__device__ __forceinline__ double trace_face(double s0, double A, double B, double sig) {
+    // 3 x and 6 x rounded once, by inline constants: 2 x + x, twice that
+    const double s3 = fma(2.0, s0, s0), ab = A + B;
+    const double s6 = 2.0 * s3 - fma(2.0, ab, ab);
+    return A + 0.5 * sig * ((B - A) + (1.0 - 2.0 / 3.0 * sig) * s6);
 }
 
-// transverse / edge corrections of one side: x - term (advective) or
-// ((x - a) - b) + c (conservative)
-template <bool CONS>
-__device__ __forceinline__ double apply3(double x, double a, double b, double c) {
-    if (CONS) return ((x - a) - b) + c;
-    return x - a;
+// the CW84 limiter (cw_limit of mx_device.H, symmetric in its two edges)
+// and the trace
+__device__ __forceinline__ double cw_trace(double s0, double A, double B, double sig) {
+    const double a = A - s0, b = s0 - B;
+    const bool flat = a * b <= 0.0;
+    const bool ca = dabs(a) >= 2.0 * dabs(b);
+    const bool cb = dabs(b) >= 2.0 * dabs(a);
+    const double s3 = fma(2.0, s0, s0);  // 3 s0
+    const double A2 = s3 - 2.0 * B, B2 = s3 - 2.0 * A;
+    const double A1 = ca ? A2 : A;
+    const double B1 = (cb && !ca) ? B2 : B;
+    return trace_face(s0, flat ? s0 : A1, flat ? s0 : B1, sig);
 }
 
-// XYF: no x- or y-boundary condition acts on the tile (the host puts a tile
-// in this class when its stencils keep clear of every physical x/y domain
-// side, or when those sides carry no boundary override), so the per-lane
-// boundary branches of those directions are left out.
-// WPE: the register budget, as waves per SIMD
-template <int PPM, bool CONS, int TX, int TY, bool XYF, int WPE>
-__global__ void __launch_bounds__(fused_nt(TX, TY)) __attribute__((amdgpu_waves_per_eu(WPE)))
+// The predictor's upwind state on the low face of a cell along a direction, s
+// the cell's S slot and F its low face value's (FST, SST: one cell along the
+// direction in the face and the S plane).
+template <int PPM, int FST, int SST>
+__device__ __forceinline__ double predict(const double* s, const double* F, bool left, bool traced,
+                                          double sig) {
+    const double* c = s + (left ? -SST : 0);
+    const double s0 = c[0];
+    double x;
+    if (PPM == 1) {
+        x = cw_trace(s0, F[0], F[left ? -FST : FST], sig);
+    } else {
+        const double* Fc = F + (left ? -FST : 0);
+        double w9[9], sm, sp;
+#pragma unroll
+        for (int o = -4; o <= 4; ++o) w9[4 + o] = (o >= -2 && o <= 2) ? c[o * SST] : 0.0;
+        cs_cell(w9, Fc[-FST], Fc[0], Fc[FST], Fc[2 * FST], 1.e-10, sm, sp);
+        x = trace_face(s0, left ? sp : sm, left ? sm : sp, sig);
+    }
+    return traced ? x : s0;
+}
+// the same with the upwind cell's boundary stencil
+template <int PPM, int D, int SST>
+__device__ __forceinline__ double predict_special(const double* s, bool left, bool traced,
+                                                  double sig, int pos, int dlo, int dhi, int bclo,
+                                                  int bchi) {
+    const double* c = s + (left ? -SST : 0);
+    double w9[9], sm, sp;
+#pragma unroll
+    for (int o = -4; o <= 4; ++o) w9[4 + o] = (o >= -1 - PPM && o <= 1 + PPM) ? c[o * SST] : 0.0;
+    ppm_edges<PPM, D>(w9, pos - (left ? 1 : 0), dlo, dhi, bclo, bchi, sm, sp);
+    const double x = trace_face(c[0], left ? sp : sm, left ? sm : sp, sig);
+    return traced ? x : c[0];
+}
+
+// MODE, the boundary conditions of the domain sides in the tile's reach: 0: each
+// side is free of overrides or extrapolates to first order (or evenly), which
+// only picks the face's upwind cell; 1: a z side may carry any; 2: any side may.
+template <int PPM, bool CONS, int TX, int TY, int MODE>
+__global__ void __launch_bounds__(fused_nt(TX, TY))
+    __attribute__((amdgpu_waves_per_eu(fused_wpe(PPM, CONS, TX, TY, MODE))))
     k_es_fused(const FBox* __restrict__ boxes, const FTile* __restrict__ tiles,
-               const FComp* __restrict__ comps, KGeom g, FArgs A, int ntile, int xmode) {
+               const FComp* __restrict__ comps, FArgs A, int ntile, int xmode) {
+    constexpr bool GEN = MODE == 2;
     constexpr int NT = fused_nt(TX, TY);
     constexpr int G = PPM == 2 ? 3 : 2;
     constexpr int W = TX + 2;
     constexpr int H = TY + 2;
-    constexpr int NE = W * H;
     constexpr int SW = W + 2 * G;
     constexpr int SH = H + 2 * G;
-    constexpr int UW = W + 1;  // x-faces per row of the x-velocity plane
-    constexpr int VH = H + 1;  // y-faces per column of the y-velocity plane
+    // x-faces per row of the x-velocity plane, y-faces per column of the
+    // y-velocity plane: the low faces of the grown tile's cells; the
+    // conservative form's divergence reads the high faces too
+    constexpr int UW = W + (CONS ? 1 : 0);
+    constexpr int VH = H + (CONS ? 1 : 0);
     constexpr int FO = PPM == 2 ? 1 : 0;
     constexpr int FXW = W + 1 + 2 * FO;  // x-face values per row
     constexpr int FYH = H + 1 + 2 * FO;  // y-face values per column
-    constexpr int NP2 = CONS ? 8 * NE : 4 * NE;
-    static_assert(NE <= NT, "tile too large for the block");
-    static_assert(FXW * H + W * FYH <= 4 * NE, "face values do not fit the pool");
+    static_assert(W * H <= NT, "tile too large for the block");
+    constexpr int NS = (SW * SH + NT - 1) / NT;
+    constexpr int NU = (UW * H + NT - 1) / NT;
+    constexpr int NV = (W * VH + NT - 1) / NT;
+    constexpr int NFX = (FXW * H + NT - 1) / NT;
+    constexpr int NFY = (W * FYH + NT - 1) / NT;
 
-    __shared__ double S[SW * SH];
-    __shared__ double UL[3][UW * H];
-    __shared__ double VL[3][W * VH];
-    __shared__ double SGX[UW * H];
-    __shared__ double SGY[W * VH];
-    __shared__ double SC[NE];
-    __shared__ double FL[NE];
-    __shared__ double P1[4 * NE];
-    __shared__ double P2[NP2];
+    // One block of LDS, so that the slots a column past the tile reads as its
+    // neighbours' lie in it: S first, whose rows keep tid - W in bounds.  Every
+    // array starts at a multiple of 512 bytes from the first, so that one
+    // two-address read reaches the same column of two of them.
+    constexpr int UP = NU * NT, VP = NV * NT;
+    constexpr int oS = 0, oU = oS + (SW * SH + 63) / 64 * 64, oV = oU + 3 * UP, oFX = oV + 3 * VP,
+                  oFY = oFX + NFX * NT, oHX = oFY + NFY * NT, oHY = oHX + NT, oTZ = oHY + NT,
+                  oXY = oTZ + NT, oYX = oXY + NT, oXZ = oYX + NT, oYZ = oXZ + NT, oEX = oYZ + NT,
+                  oEY = oEX + NT, oFL = oEY + NT, oBB = oFL + NT, oSC = oBB + (CONS ? 2 * NT : 0),
+                  oCZ = oSC + (CONS ? 2 * NT : 0), oEnd = oCZ + (CONS ? NT : 0) + W + 2;
+    __shared__ double lds[oEnd];
+    double* S = lds + oS;
+    double* FX = lds + oFX;
+    double* FY = lds + oFY;
+    double* HX = lds + oHX;
+    double* HY = lds + oHY;
+    double* TZ = lds + oTZ;
+    double* XY = lds + oXY;
+    double* YX = lds + oYX;
+    double* XZ = lds + oXZ;
+    double* YZ = lds + oYZ;
+    double* EX = lds + oEX;
+    double* EY = lds + oEY;
+    double* FL = lds + oFL;
+    double* CZ = lds + oCZ;
 
     // xmode 1, 2: the XCD-aware orders of xcd_tile over a 1-D grid; 0: tile
     // blockIdx.x and component blockIdx.z
     int tix = blockIdx.x, vc = blockIdx.z;
     if (xmode != 0 && !xcd_tile(ntile, A.num_comp, xmode, tix, vc)) return;
     const FTile tl = tiles[tix];
-    const int bid = tl.box;
-    const int blo0 = boxes[bid].lo[0], blo1 = boxes[bid].lo[1], blo2 = boxes[bid].lo[2];
-    const int bhi0 = boxes[bid].hi[0], bhi1 = boxes[bid].hi[1], bhi2 = boxes[bid].hi[2];
-    const int tx = tl.tx;
-    const int ty = tl.ty;
-    const int tzc = tl.tzc;
-    const int X0 = blo0 + tx * TX;
-    const int Y0 = blo1 + ty * TY;
-    const int nx = min(TX, bhi0 - X0 + 1);
-    const int ny = min(TY, bhi1 - Y0 + 1);
-    const int z0 = blo2 + tzc * A.tz;
-    const int z1 = min(z0 + A.tz - 1, bhi2);
-    const bool last_x = (X0 + nx - 1 == bhi0);
-    const bool last_y = (Y0 + ny - 1 == bhi1);
-    const bool last_z = (z1 == bhi2);
+    const FBox& B = boxes[tl.box];
+    const int X0 = tl.x0, Y0 = tl.y0, nx = tl.nx, ny = tl.ny;
+    const int z0 = tl.z0, z1 = tl.z0 + tl.nz - 1;
+    const bool last_x = X0 + nx - 1 == B.hi[0];
+    const bool last_y = Y0 + ny - 1 == B.hi[1];
+    const bool last_z = z1 == B.hi[2];
 
     const int comp = comps[vc].comp;
     const int flux = comps[vc].flux;
-    const int bcx0 = comps[vc].bclo[0], bcx1 = comps[vc].bchi[0];
-    const int bcy0 = comps[vc].bclo[1], bcy1 = comps[vc].bchi[1];
-    const int bcz0 = comps[vc].bclo[2], bcz1 = comps[vc].bchi[2];
-    const int dlx = boxes[bid].domlo[0], dhx = boxes[bid].domhi[0];
-    const int dly = boxes[bid].domlo[1], dhy = boxes[bid].domhi[1];
-    const int dlz = boxes[bid].domlo[2], dhz = boxes[bid].domhi[2];
+    const int* bcl = comps[vc].bclo;
+    const int* bch = comps[vc].bchi;
 
-    // views (the strides fit 32 bits; checked on the host)
-    const DA sv = boxes[bid].s;
-    const DA fv = boxes[bid].fo;
-    const DA uv = boxes[bid].um[0];
-    const DA vv = boxes[bid].um[1];
-    const DA wv = boxes[bid].um[2];
-    const DA e0 = boxes[bid].se[0];
-    const DA e1 = boxes[bid].se[1];
-    const DA e2 = boxes[bid].se[2];
-    const int sjs = (int)sv.js, sks = (int)sv.ks;
-    const int ujs = (int)uv.js, uks = (int)uv.ks;
-    const int vjs = (int)vv.js, vks = (int)vv.ks;
+    const double dt = A.dt, eps = A.rel_eps, dt2 = A.dt2, dt3 = A.dt3;
+    const double tfx = uniform(A.tf / B.h[0].d), tfy = uniform(A.tf / B.h[1].d),
+                 tfz = uniform(A.tf / B.h[2].d);
+    const double efx = uniform(A.ef / B.h[0].d), efy = uniform(A.ef / B.h[1].d),
+                 efz = uniform(A.ef / B.h[2].d);
+    double dt2hx = 0.0, dt2hy = 0.0, dt2hz = 0.0;
+    if (CONS) {
+        dt2hx = uniform(dt2 / B.h[0].d);
+        dt2hy = uniform(dt2 / B.h[1].d);
+        dt2hz = uniform(dt2 / B.h[2].d);
+    }
 
     const int tid = threadIdx.x;
     const int a = tid % W;  // local column: cell (X0 + a - 1, Y0 + b - 1)
     const int b = tid / W;
-    const bool col = (tid < NE) && (a <= nx + 1) && (b <= ny + 1);
     const int I = X0 + a - 1;
     const int J = Y0 + b - 1;
     const int si = (a + G) + (b + G) * SW;
-    const int ui = a + b * UW;
-    const int vi = a + b * W;
+    const int ui = CONS ? a + b * UW : tid;
+    const bool inx = a >= 1 && a <= nx, iny = b >= 1 && b <= ny;
+    const bool st_x = a >= 1 && iny && (a <= nx || (last_x && a == nx + 1));
+    const bool st_y = b >= 1 && inx && (b <= ny || (last_y && b == ny + 1));
+    const bool st_z = inx && iny;
+    const Side dx(I, B.domlo[0], B.domhi[0], bcl[0], bch[0], A.is_vel && comp == 0);
+    const Side dy(J, B.domlo[1], B.domhi[1], bcl[1], bch[1], A.is_vel && comp == 1);
+    // the z-faces on acting sides
+    const int zlo = side_kind(bcl[2]) ? B.domlo[2] : INT_MIN;
+    const int zhi = side_kind(bch[2]) ? B.domhi[2] + 1 : INT_MIN;
+    // z-face q may need more than its upwind cell: a boundary stencil, a fixed
+    // value or a clamp.  Uniform, and rare: the branches it guards read the
+    // table and the column's cells again.
+    const bool zgl = tl.zgen & 1, zgh = tl.zgen & 2;
+    auto z_general = [&](int q) {
+        return MODE > 0 && ((zgl && q <= B.domlo[2] + 3) || (zgh && q >= B.domhi[2] - 2));
+    };
+    auto side_z = [&](int q) {
+        cbox* Bf = fresh(&B);
+        return Side(q, Bf->domlo[2], Bf->domhi[2], bcl[2], bch[2], A.is_vel && comp == 2);
+    };
 
-    const double dt = g.dt;
-    const double rel_eps = g.rel_eps;
-    const double dt2 = 0.5 * dt;
-    const double dt3 = dt / 3.0;
-    const double dt4 = 0.25 * dt;
-    const double dt6 = dt / 6.0;
-    const double hx = boxes[bid].dx[0], hy = boxes[bid].dx[1], hz = boxes[bid].dx[2];
-    // per-direction factors of the transverse (t) and edge (e) terms
-    const double tfx = CONS ? dt3 / hx : dt6 / hx;
-    const double tfy = CONS ? dt3 / hy : dt6 / hy;
-    const double tfz = CONS ? dt3 / hz : dt6 / hz;
-    const double efx = CONS ? dt2 / hx : dt4 / hx;
-    const double efy = CONS ? dt2 / hy : dt4 / hy;
-    const double efz = CONS ? dt2 / hz : dt4 / hz;
-    const double dt2hx = dt2 / hx, dt2hy = dt2 / hy, dt2hz = dt2 / hz;
-    const bool vn0 = A.is_vel && comp == 0;
-    const bool vn1 = A.is_vel && comp == 1;
-    const bool vn2 = A.is_vel && comp == 2;
-
-    // plane pointers (block-uniform) at plane z0 - 1
-    gcd* sPl = (gcd*)sv.p + sv.off(X0 - 1 - G, Y0 - 1 - G, z0 - 1, comp);
-    gcd* uPl = (gcd*)uv.p + uv.off(X0 - 1, Y0 - 1, z0 - 1);
-    gcd* vPl = (gcd*)vv.p + vv.off(X0 - 1, Y0 - 1, z0 - 1);
-    // column pointers
-    gcd* sCol = (gcd*)sv.p;
-    gcd* fCol = (gcd*)fv.p;
-    gcd* wCol = (gcd*)wv.p;
-    gd* e0Col = (gd*)e0.p;
-    gd* e1Col = (gd*)e1.p;
-    gd* e2Col = (gd*)e2.p;
-    if (col) {
-        sCol += sv.off(I, J, z0 - 1 + G, comp);  // next z-window load: s(q + G)
-        fCol += fv.off(I, J, z0 - 1, comp);
-        wCol += wv.off(I, J, z0 - 1);
-        e0Col += e0.off(I, J, z0 - 1, comp);
-        e1Col += e1.off(I, J, z0 - 1, comp);
-        e2Col += e2.off(I, J, z0 - 1, comp);
-    }
-    const int fks = (int)fv.ks, wks = (int)wv.ks;
-    const int e0ks = (int)e0.ks, e1ks = (int)e1.ks, e2ks = (int)e2.ks;
-
-    // column state
-    double v[9];
-    for (int jj = 0; jj < 9; ++jj) v[jj] = 0.0;
-    double w_q = 0.0, w_p = 0.0, w_hi = 0.0, sig_lo = 0.0;
-    double fo_q = 0.0, fo_p = 0.0;
-    double zf0 = 0.0, zf1 = 0.0, zf2 = 0.0, zsl = 0.0;  // z face values / slope queue
-    double Ipz_prev = 0.0, slz = 0.0, srz = 0.0, hz_q = 0.0, hz_p = 0.0;
-    double slx = 0.0, srx = 0.0, sly = 0.0, sry = 0.0;
-    double slx_p = 0.0, srx_p = 0.0, sly_p = 0.0, sry_p = 0.0;
-    double tx_q = 0.0, tx_p = 0.0, ty_q = 0.0, ty_p = 0.0;     // own transverse terms
-    double cx_q = 0.0, cx_p = 0.0, cy_q = 0.0, cy_p = 0.0;     // conservative parts
-    double bq = 0.0, bp = 0.0;
-    double tzx_q = 0.0, tzx_p = 0.0, tzy_q = 0.0, tzy_p = 0.0;  // simhzx, simhzy
-    double exy_q = 0.0, exy_p = 0.0, eyx_q = 0.0, eyx_p = 0.0;  // own edge terms
-    if (col) {
-        for (int jj = 5 - G; jj <= 4 + G; ++jj) v[jj] = sv(I, J, z0 - 6 + jj, comp);
-        w_q = wv(I, J, z0 - 1);
-        sig_lo = dabs(w_q) * dt / hz;
-    }
-    int slot_q = 0, slot_p = 2;
-
-    // Plane q + 1's loads are issued during step q and land in registers
-    // (the barriers wait for LDS traffic only), so the global-memory latency
-    // overlaps the step's work.  Each thread owns fixed slots of the staged
-    // planes: s (NS per thread), the x- and y-velocities (NU, NV).
-    constexpr int NS = (SW * SH + NT - 1) / NT;
-    constexpr int NU = (UW * H + NT - 1) / NT;
-    constexpr int NV = (W * VH + NT - 1) / NT;
-    bool okS[NS], okU[NU], okV[NV];
-    int offS[NS], offU[NU], offV[NV];
+    // byte offsets within a plane of the tile's arrays; a column past the
+    // tile takes the tile's last one
+    const DA sv = B.s, fv = B.fo, uv = B.um[0], vv = B.um[1], wv = B.um[2];
+    const int ac = min(a, nx + 1), bc = min(b, ny + 1);
+    const unsigned sjs = (unsigned)sv.js * 8u;
+    const unsigned oCol = (unsigned)(ac + G) * 8u + (unsigned)(bc + G) * sjs;
+    const unsigned oF = (unsigned)ac * 8u + (unsigned)bc * (unsigned)fv.js * 8u;
+    const unsigned oW = (unsigned)ac * 8u + (unsigned)bc * (unsigned)wv.js * 8u;
+    const unsigned oE0 = (unsigned)ac * 8u + (unsigned)bc * (unsigned)B.se[0].js * 8u;
+    const unsigned oE1 = (unsigned)ac * 8u + (unsigned)bc * (unsigned)B.se[1].js * 8u;
+    const unsigned oE2 = (unsigned)ac * 8u + (unsigned)bc * (unsigned)B.se[2].js * 8u;
+    // each thread's slots of the staged planes (an item past the plane is the
+    // thread's first again)
+    unsigned offS[NS], offU[NU], offV[NV];
+    int slS[NS];
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
-        const int idx = tid + k * NT;
-        const int sx = idx % SW, sy = idx / SW;
-        okS[k] = idx < SW * SH && sx <= nx + 1 + 2 * G && sy <= ny + 1 + 2 * G;
-        offS[k] = sx + sy * sjs;
+        const int idx = tid + k * NT < SW * SH ? tid + k * NT : tid;
+        slS[k] = idx;
+        offS[k] = (unsigned)min(idx % SW, nx + 1 + 2 * G) * 8u +
+                  (unsigned)min(idx / SW, ny + 1 + 2 * G) * sjs;
     }
 #pragma unroll
     for (int k = 0; k < NU; ++k) {
         const int idx = tid + k * NT;
-        const int f = idx % UW, r = idx / UW;
-        okU[k] = idx < UW * H && f <= nx + 2 && r <= ny + 1;
-        offU[k] = f + r * ujs;
+        offU[k] = (unsigned)min(idx % UW, nx + 2) * 8u +
+                  (unsigned)min(idx / UW, ny + 1) * (unsigned)uv.js * 8u;
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int idx = tid + k * NT;
-        const int cc = idx % W, r = idx / W;
-        okV[k] = idx < W * VH && cc <= nx + 1 && r <= ny + 2;
-        offV[k] = cc + r * vjs;
+        offV[k] = (unsigned)min(idx % W, nx + 1) * 8u +
+                  (unsigned)min(idx / W, ny + 2) * (unsigned)vv.js * 8u;
     }
+    // S slot of this thread's x- and y-face items
+    int fxi[NFX], fyi[NFY];
+#pragma unroll
+    for (int k = 0; k < NFX; ++k) {
+        const int idx = min(tid + k * NT, FXW * H - 1);
+        fxi[k] = (idx % FXW - FO + G) + (idx / FXW + G) * SW;
+    }
+#pragma unroll
+    for (int k = 0; k < NFY; ++k) {
+        const int idx = min(tid + k * NT, W * FYH - 1);
+        fyi[k] = (idx % W + G) + (idx / W - FO + G) * SW;
+    }
+
+    // Plane bases (block-uniform).  Loads: s, u, v, w and the force of the
+    // next plane to load, s also G planes further for the column window; stores: the edge
+    // states' plane.
+    gcc* sN = (gcc*)sv.p + 8 * sv.off(X0 - 1 - G, Y0 - 1 - G, z0 - 1, comp);
+    gcc* uN = (gcc*)uv.p + 8 * uv.off(X0 - 1, Y0 - 1, z0 - 1);
+    gcc* vN = (gcc*)vv.p + 8 * vv.off(X0 - 1, Y0 - 1, z0 - 1);
+    gcc* wN = (gcc*)wv.p + 8 * wv.off(X0 - 1, Y0 - 1, z0 - 1);
+    gcc* fN = (gcc*)fv.p + 8 * fv.off(X0 - 1, Y0 - 1, z0 - 1, comp);
+    gcc* sC = sN + G * B.ks[0];
+    gc* e0P = (gc*)B.se[0].p + 8 * B.se[0].off(X0 - 1, Y0 - 1, z0 - 3, comp);
+    gc* e1P = (gc*)B.se[1].p + 8 * B.se[1].off(X0 - 1, Y0 - 1, z0 - 3, comp);
+    gc* e2P = (gc*)B.se[2].p + 8 * B.se[2].off(X0 - 1, Y0 - 1, z0 - 2, comp);
+
+    // column state of step q, moved on to q + 1 in phase 1: v[jj] =
+    // s(q - 4 + jj); w_p, w_q, w_hi: w on z-faces q - 1, q, q + 1; p..: loaded
+    // for the next step
+    double v[9];
+#pragma unroll
+    for (int jj = 0; jj < 9; ++jj) v[jj] = 0.0;
+#pragma unroll
+    for (int jj = 4 - G; jj < 4 + G; ++jj) v[jj + 1] = gload(sN + (jj - 4) * B.ks[0], oCol);
+    double w_p = 0.0, w_q = 0.0, w_hi = gload(wN, oW), fo_p = 0.0, fo_q = 0.0;
+    double pcs = gload(sC, oCol), pw = gload(wN + B.ks[4], oW), pf = gload(fN, oF);
+    // z face values q - 1, q, q + 1 at phase 2, and the slope of cell q
+    double zf0 = 0.0, zf1 = 0.0, zf2 = 0.0, zsl = 0.0;
+    double sig_lo = 0.0, Ipz_prev = 0.0;
+    double sx = 0.0, sy = 0.0, sz = 0.0, sx_p = 0.0, sy_p = 0.0, sz_p = 0.0;
+    double tx_p = 0.0, ty_p = 0.0, cx_p = 0.0, cy_p = 0.0, bp = 0.0;
+    double tzx_p = 0.0, tzy_p = 0.0, exy_p = 0.0, eyx_p = 0.0;
+    if (PPM == 1) {
+        const double d0 = vl_slope(v[3], v[4], v[5]);
+        zsl = vl_slope(v[4], v[5], v[6]);
+        zf1 = face1(v[4], v[5], d0, zsl);  // face z0 - 1
+    } else {
+        zf0 = cs_face(v[2], v[3], v[4], v[5]);
+        zf1 = cs_face(v[3], v[4], v[5], v[6]);
+        zf2 = cs_face(v[4], v[5], v[6], v[7]);
+        sig_lo = div_by(dabs(w_hi) * dt, B.h[2]);
+    }
+
+    // Plane q + 1's loads are issued at the start of step q and land in
+    // registers (the barriers wait for LDS traffic only); phase 3 puts them
+    // in LDS.  Each thread owns fixed slots of the staged planes.
     double pS[NS], pU[NU], pV[NV];
-    double pcs = 0.0, pw = 0.0, pf = 0.0;
-    // plane z0 - 1
+    auto load_planes = [&](gcc* s, gcc* u, gcc* vp) {
 #pragma unroll
-    for (int k = 0; k < NS; ++k) pS[k] = okS[k] ? sPl[offS[k]] : 0.0;
+        for (int k = 0; k < NS; ++k) pS[k] = gload(s, offS[k]);
 #pragma unroll
-    for (int k = 0; k < NU; ++k) pU[k] = okU[k] ? uPl[offU[k]] : 0.0;
+        for (int k = 0; k < NU; ++k) pU[k] = gload(u, offU[k]);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) pV[k] = okV[k] ? vPl[offV[k]] : 0.0;
-    if (col) {
-        pcs = *sCol;
-        pw = wCol[wks];
-        pf = *fCol;
-    }
+        for (int k = 0; k < NV; ++k) pV[k] = gload(vp, offV[k]);
+    };
+    auto stage_planes = [&](int slot) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) S[(k + 1) * NT <= SW * SH ? tid + k * NT : slS[k]] = pS[k];
+#pragma unroll
+        for (int k = 0; k < NU; ++k) lds[oU + slot * UP + tid + k * NT] = pU[k];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) lds[oV + slot * VP + tid + k * NT] = pV[k];
+    };
+    // plane k of s (rare paths)
+    auto s_plane = [&](int k) {
+        cbox* Bf = fresh(&B);
+        return (gcc*)Bf->s.p + 8 * ((long long)(X0 - 1 - G - Bf->s.b0) +
+                                    (long long)(Y0 - 1 - G - Bf->s.b1) * Bf->s.js +
+                                    (long long)(k - Bf->s.b2) * Bf->s.ks +
+                                    (long long)comp * Bf->s.ns);
+    };
+    load_planes(sN, uN, vN);
+    stage_planes(0);
+    int slot_q = 0, slot_p = 2, slot_o = 1;  // planes q, q - 1, q - 2 (then q + 1)
+    // on to the next plane; the loads stay at plane z1 + 1 (a step past it loads
+    // it again: conditional loads would leave the compiler's wait counters open
+    // and stall on every load in flight)
+    auto advance = [&](bool more) {
+        __attribute__((address_space(4))) const long long* ks = fresh(&B)->ks;
+        if (more) {
+            sN += ks[0];
+            sC += ks[0];
+            fN += ks[1];
+            uN += ks[2];
+            vN += ks[3];
+            wN += ks[4];
+        }
+        e0P += ks[5];
+        e1P += ks[6];
+        e2P += ks[7];
+    };
+    // The edge states of step r = q - 1: x- and y-faces of plane r - 1, z-face
+    // r, from the column state of step r (at the first two steps, with nothing to
+    // store, of whatever LDS holds).
+    auto edges = [&](int q) {
+        const double* ULp = lds + oU + slot_p * UP;  // plane r
+        const double* VLp = lds + oV + slot_p * VP;
+        const double* ULo = lds + oU + slot_o * UP;  // plane r - 1
+        const double* VLo = lds + oV + slot_o * VP;
+        const double* SCo = lds + oSC + (CONS ? (q & 1) * NT : 0);  // s, plane r - 1
+        const double u0 = ULo[ui], v0 = VLo[tid];
+        const Face fx(u0, eps, dx.lo, dx.hi), fy(v0, eps, dy.lo, dy.hi),
+            fz(w_q, eps, q - 1 == zlo, q - 1 == zhi);
+        auto edge_x = [&](double s, int o) {
+            const int t = tid + o;
+            const double y1 = VLo[t + W], y0 = VLo[t], h1 = YZ[t + W], h0 = YZ[t];
+            double x = s - (CONS ? efy * (h1 * y1 - h0 * y0) : efy * (y1 + y0) * (h1 - h0));
+            x = x - EY[t];
+            if (CONS) x = x - dt2hx * SCo[t] * (ULo[ui + o + 1] - ULo[ui + o]);
+            return x + dt2 * FL[t];
+        };
+        auto edge_y = [&](double s, int n) {
+            const int t = tid + n * W, u = ui + n * UW;
+            const double x1 = ULo[u + 1], x0 = ULo[u], h1 = XZ[t + 1], h0 = XZ[t];
+            double x = s - (CONS ? efx * (h1 * x1 - h0 * x0) : efx * (x1 + x0) * (h1 - h0));
+            x = x - EX[t];
+            if (CONS) x = x - dt2hy * SCo[t] * (VLo[t + W] - VLo[t]);
+            return x + dt2 * FL[t];
+        };
+        const double a1 = ULp[ui + 1], a0 = ULp[ui], b1 = VLp[tid + W], b0 = VLp[tid];
+        const double x1 = XY[tid + 1], x0 = XY[tid], y1 = YX[tid + W], y0 = YX[tid];
+        const double exy = CONS ? efx * (x1 * a1 - x0 * a0) : efx * (a1 + a0) * (x1 - x0);
+        const double eyx = CONS ? efy * (y1 * b1 - y0 * b0) : efy * (b1 + b0) * (y1 - y0);
+        auto edge_z = [&](double s, bool left) {
+            double x = s - (left ? exy_p : exy);
+            x = x - (left ? eyx_p : eyx);
+            if (CONS) x = x - dt2hz * (left ? v[3] : v[4]) * (left ? w_q - w_p : w_hi - w_q);
+            return x + dt2 * (left ? fo_p : fo_q);
+        };
+        double rx = edge_x(sx_p, fx.left ? -1 : 0);
+        double ry = edge_y(sy_p, fy.left ? -1 : 0);
+        double rz = edge_z(sz, fz.left);
+        if (fx.both | fy.both | fz.both) {
+            gcc* row = s_plane(q - 2);
+            if (fx.both)
+                rx = 0.5 * (edge_x(gload(row, oCol - 8u), -1) + edge_x(gload(row, oCol), 0));
+            if (fy.both)
+                ry = 0.5 * (edge_y(gload(row, oCol - sjs), -1) + edge_y(gload(row, oCol), 0));
+            if (fz.both) rz = 0.5 * (edge_z(v[3], true) + edge_z(v[4], false));
+        }
+        if (GEN) {
+            rx = dx.set(rx, sx_p);
+            ry = dy.set(ry, sy_p);
+        }
+        if (z_general(q - 1)) rz = side_z(q - 1).set(rz, sz);
+        exy_p = exy;
+        eyx_p = eyx;
+        if (q >= z0 + 2) {
+            if (st_x) gstore(e0P, oE0, rx);
+            if (st_y) gstore(e1P, oE1, ry);
+            if (flux) {
+                if (st_x) flux_store(B, 0, I, J, q - 2, comp, flux, u0, rx);
+                if (st_y) flux_store(B, 1, I, J, q - 2, comp, flux, v0, ry);
+            }
+        }
+        if (q > z0 && (q <= z1 + 1 || last_z) && st_z) {
+            gstore(e2P, oE2, rz);
+            if (flux) flux_store(B, 2, I, J, q - 1, comp, flux, w_q, rz);
+        }
+    };
+    // w and s of plane z0 are loaded: step z0 - 1 loads the planes after
+    sN += B.ks[0];
+    sC += B.ks[0];
+    fN += B.ks[1];
+    uN += B.ks[2];
+    vN += B.ks[3];
+    wN += 2 * B.ks[4];
+    __syncthreads();
 
     for (int q = z0 - 1; q <= z1 + 1; ++q) {
-        const bool zface = q >= z0;        // z-face q is in the chunk's range
-        const bool pplane = q >= z0 + 1;   // plane p = q - 1 is a chunk plane
-        const bool first = q == z0 - 1;
-        double* ULq = UL[slot_q];
-        double* VLq = VL[slot_q];
-        const double* ULp = UL[slot_p];
-        const double* VLp = VL[slot_p];
+        const double* ULq = lds + oU + slot_q * UP;
+        const double* VLq = lds + oV + slot_q * VP;
+        const double* ULp = lds + oU + slot_p * UP;
+        const double* VLp = lds + oV + slot_p * VP;
+        load_planes(sN, uN, vN);
 
-        // ---- A: stage plane q (loaded during the previous step); shift the
-        //      column window; issue the loads of plane q + 1
+        // ---- 1a: the edge states of step q - 1; the column state moves on
+        edges(q);
 #pragma unroll
-        for (int k = 0; k < NS; ++k)
-            if (okS[k]) S[tid + k * NT] = pS[k];
+        for (int jj = 0; jj < 8; ++jj) v[jj] = v[jj + 1];
+        v[4 + G] = pcs;
+        sx_p = sx;
+        sy_p = sy;
+        sz_p = sz;
+        w_p = w_q;
+        w_q = w_hi;
+        w_hi = pw;
+        fo_p = fo_q;
+        fo_q = pf;
+        pcs = gload(sC, oCol);
+        pw = gload(wN, oW);
+        pf = gload(fN, oF);
+
+        // ---- 1b: PPM face values of plane q
 #pragma unroll
-        for (int k = 0; k < NU; ++k)
-            if (okU[k]) {
-                ULq[tid + k * NT] = pU[k];
-                SGX[tid + k * NT] = dabs(pU[k]) * dt / hx;
-            }
-#pragma unroll
-        for (int k = 0; k < NV; ++k)
-            if (okV[k]) {
-                VLq[tid + k * NT] = pV[k];
-                SGY[tid + k * NT] = dabs(pV[k]) * dt / hy;
-            }
-        if (col) {
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) v[jj] = v[jj + 1];
-            v[4 + G] = pcs;
-            w_hi = pw;
-            fo_q = pf;
+        for (int k = 0; k < NFX; ++k) {
+            const double* s = S + fxi[k];  // face between s[-1] and s[0]
+            FX[tid + k * NT] = PPM == 1 ? face1(s[-1], s[0], vl_slope(s[-2], s[-1], s[0]),
+                                                vl_slope(s[-1], s[0], s[1]))
+                                        : cs_face(s[-2], s[-1], s[0], s[1]);
         }
-        if (q <= z1) {
-            sPl += sks;
-            uPl += uks;
-            vPl += vks;
 #pragma unroll
-            for (int k = 0; k < NS; ++k)
-                if (okS[k]) pS[k] = sPl[offS[k]];
-#pragma unroll
-            for (int k = 0; k < NU; ++k)
-                if (okU[k]) pU[k] = uPl[offU[k]];
-#pragma unroll
-            for (int k = 0; k < NV; ++k)
-                if (okV[k]) pV[k] = vPl[offV[k]];
-            if (col) {
-                sCol += sks;
-                fCol += fks;
-                pcs = *sCol;
-                pw = wCol[2 * wks];
-                pf = *fCol;
-            }
+        for (int k = 0; k < NFY; ++k) {
+            const double* s = S + fyi[k];
+            FY[tid + k * NT] =
+                PPM == 1 ? face1(s[-SW], s[0], vl_slope(s[-2 * SW], s[-SW], s[0]),
+                                 vl_slope(s[-SW], s[0], s[SW]))
+                         : cs_face(s[-2 * SW], s[-SW], s[0], s[SW]);
         }
+        cbox* Bq = fresh(&B);
+        const DivBy hx{Bq->h[0].d, Bq->h[0].r, Bq->h[0].rl}, hy{Bq->h[1].d, Bq->h[1].r, Bq->h[1].rl},
+            hz{Bq->h[2].d, Bq->h[2].r, Bq->h[2].rl};
         __syncthreads();
 
-        // ---- B1: PPM face values of plane q; PPM of cell q in z
+        // ---- 2: the predictor's upwind states on the low faces of cell q
+        const double ux = ULq[ui], vy = VLq[tid];
+        const Face fx(ux, eps, dx.lo, dx.hi), fy(vy, eps, dy.lo, dy.hi),
+            fz(w_q, eps, q == zlo, q == zhi);
         {
-            double* FX = P1;
-            double* FY = P1 + FXW * H;
-            for (int idx = tid; idx < FXW * H; idx += NT) {
-                const int f = idx % FXW - FO, r = idx / FXW;  // face f: cells f-1 | f
-                if (f <= nx + 2 + FO && r <= ny + 1) {
-                    const double* sr = S + (f + G) + (r + G) * SW;
-                    if (PPM == 1) {
-                        const double sa2 = sr[-2], sa = sr[-1], sb = sr[0], sb2 = sr[1];
-                        FX[idx] = face1(sa, sb, vl_slope(sa2, sa, sb), vl_slope(sa, sb, sb2));
-                    } else {
-                        FX[idx] = cs_face(sr[-2], sr[-1], sr[0], sr[1]);
-                    }
-                }
-            }
-            for (int idx = tid; idx < W * FYH; idx += NT) {
-                const int c = idx % W, f = idx / W - FO;  // face f: cells f-1 | f
-                if (c <= nx + 1 && f <= ny + 2 + FO) {
-                    const double* sr = S + (c + G) + (f + G) * SW;
-                    if (PPM == 1) {
-                        const double sa2 = sr[-2 * SW], sa = sr[-SW], sb = sr[0], sb2 = sr[SW];
-                        FY[idx] = face1(sa, sb, vl_slope(sa2, sa, sb), vl_slope(sa, sb, sb2));
-                    } else {
-                        FY[idx] = cs_face(sr[-2 * SW], sr[-SW], sr[0], sr[SW]);
-                    }
-                }
-            }
-        }
-        double Ipz = 0.0, Imz = 0.0;
-        if (col) {
-            SC[tid] = v[3];
-            FL[tid] = fo_p;
-            double sm, sp;
+            const bool px = fx.traced, py = fy.traced, pz = fz.traced;
+            const double gx = div_by(dabs(ux) * dt, hx), gy = div_by(dabs(vy) * dt, hy);
+            sx = predict<PPM, 1, 1>(S + si, FX + (a + FO) + b * FXW, fx.left, px, gx);
+            sy = predict<PPM, W, SW>(S + si, FY + a + (b + FO) * W, fy.left, py, gy);
             if (PPM == 1) {
-                // zf0 = face q, zsl = slope(q); new: slope(q+1), face q+1
-                if (first) {
-                    const double d0 = vl_slope(v[2], v[3], v[4]);
-                    zsl = vl_slope(v[3], v[4], v[5]);
-                    zf0 = face1(v[3], v[4], d0, zsl);
-                }
                 const double d1 = vl_slope(v[4], v[5], v[6]);
-                zf1 = face1(v[4], v[5], zsl, d1);
+                zf2 = face1(v[4], v[5], zsl, d1);
                 zsl = d1;
-                sm = zf0;
-                sp = zf1;
-                cw_limit(v[4], sm, sp);
-            } else {
-                // zf0, zf1, zf2 = faces q-1, q, q+1; new: face q+2
-                if (first) {
-                    zf0 = cs_face(v[1], v[2], v[3], v[4]);
-                    zf1 = cs_face(v[2], v[3], v[4], v[5]);
-                    zf2 = cs_face(v[3], v[4], v[5], v[6]);
+                const double s0 = fz.left ? v[3] : v[4];
+                const double gz = div_by(dabs(w_q) * dt, hz);
+                const double t = cw_trace(s0, zf1, fz.left ? zf0 : zf2, gz);
+                sz = pz ? t : s0;
+                zf0 = zf1;
+                zf1 = zf2;
+                if (z_general(q)) {
+                    cbox* Bf = fresh(&B);
+                    const int dl = Bf->domlo[2], dh = Bf->domhi[2];
+                    const int pos = q - (fz.left ? 1 : 0);
+                    if (ppm_special<PPM>(pos, dl, dh, bcl[2], bch[2])) {
+                        double w9[9], sm, sp;
+#pragma unroll
+                        for (int o = 0; o < 9; ++o)
+                            w9[o] = o >= 2 && o <= 6
+                                        ? (fz.left ? gload(s_plane(q - 5 + o), oCol)
+                                                   : gload(s_plane(q - 4 + o), oCol))
+                                        : 0.0;
+                        ppm_edges<PPM, 2>(w9, pos, dl, dh, bcl[2], bch[2], sm, sp);
+                        const double x =
+                            trace_face(s0, fz.left ? sp : sm, fz.left ? sm : sp, gz);
+                        sz = pz ? x : s0;
+                    }
                 }
+            } else {
+                double sm, sp, Ipz, Imz;
                 const double f3 = cs_face(v[4], v[5], v[6], v[7]);
                 cs_cell(v, zf0, zf1, zf2, f3, 1.e-10, sm, sp);
                 zf0 = zf1;
                 zf1 = zf2;
                 zf2 = f3;
-            }
-            if (ppm_special<PPM>(q, dlz, dhz, bcz0, bcz1))
-                ppm_edges<PPM, 2>(v, q, dlz, dhz, bcz0, bcz1, sm, sp);
-            if (PPM == 1) zf0 = zf1;
-            const double sig_hi = dabs(w_hi) * dt / hz;
-            trace_sig(v[4], sm, sp, w_hi, w_q, sig_hi, sig_lo, rel_eps, Ipz, Imz);
-            sig_lo = sig_hi;
-            if (zface) {
-                slz = Ipz_prev;
-                srz = Imz;
-                bc_pair(q, dlz, dhz, bcz0, bcz1, vn2, v[3], v[4], slz, srz);
-                hz_q = upwind(slz, srz, w_q, 0.0);
-            }
-            Ipz_prev = Ipz;
-        }
-        __syncthreads();
-
-        // ---- B2: PPM of plane q in x and y
-        if (col) {
-            const double* FX = P1;
-            const double* FY = P1 + FXW * H;
-            double sm, sp, Ip, Im;
-            double w9[9];
-#pragma unroll
-            for (int o = -4; o <= 4; ++o) w9[4 + o] = (o >= -G && o <= G) ? S[si + o] : 0.0;
-            const int fx = (a + FO) + b * FXW;
-            if (PPM == 1) {
-                sm = FX[fx];
-                sp = FX[fx + 1];
-                cw_limit(w9[4], sm, sp);
-            } else {
-                cs_cell(w9, FX[fx - 1], FX[fx], FX[fx + 1], FX[fx + 2], 1.e-10, sm, sp);
-            }
-            if (!XYF && ppm_special<PPM>(I, dlx, dhx, bcx0, bcx1))
-                ppm_edges<PPM, 0>(w9, I, dlx, dhx, bcx0, bcx1, sm, sp);
-            trace_sig(w9[4], sm, sp, ULq[ui + 1], ULq[ui], SGX[ui + 1], SGX[ui], rel_eps, Ip,
-                      Im);
-            P2[tid] = Ip;
-            P2[NE + tid] = Im;
-#pragma unroll
-            for (int o = -4; o <= 4; ++o) w9[4 + o] = (o >= -G && o <= G) ? S[si + o * SW] : 0.0;
-            const int fy = a + (b + FO) * W;
-            if (PPM == 1) {
-                sm = FY[fy];
-                sp = FY[fy + W];
-                cw_limit(w9[4], sm, sp);
-            } else {
-                cs_cell(w9, FY[fy - W], FY[fy], FY[fy + W], FY[fy + 2 * W], 1.e-10, sm, sp);
-            }
-            if (!XYF && ppm_special<PPM>(J, dly, dhy, bcy0, bcy1))
-                ppm_edges<PPM, 1>(w9, J, dly, dhy, bcy0, bcy1, sm, sp);
-            trace_sig(w9[4], sm, sp, VLq[vi + W], VLq[vi], SGY[vi + W], SGY[vi], rel_eps, Ip,
-                      Im);
-            P2[2 * NE + tid] = Ip;
-            P2[3 * NE + tid] = Im;
-        }
-        __syncthreads();
-
-        // ---- C: predictor and upwind states on the x- and y-faces of plane q
-        if (col && a >= 1) {
-            slx = P2[tid - 1];
-            srx = P2[NE + tid];
-            if (!XYF) bc_pair(I, dlx, dhx, bcx0, bcx1, vn0, S[si - 1], S[si], slx, srx);
-            P1[tid] = upwind(slx, srx, ULq[ui], 0.0);
-        }
-        if (col && b >= 1) {
-            sly = P2[2 * NE + tid - W];
-            sry = P2[3 * NE + tid];
-            if (!XYF) bc_pair(J, dly, dhy, bcy0, bcy1, vn1, S[si - SW], S[si], sly, sry);
-            P1[NE + tid] = upwind(sly, sry, VLq[vi], 0.0);
-        }
-        __syncthreads();
-
-        // ---- D1: per-cell transverse terms
-        if (col) {
-            const double ux1 = ULq[ui + 1], ux0 = ULq[ui];
-            const double vy1 = VLq[vi + W], vy0 = VLq[vi];
-            if (CONS) {
-                double dv = ux1 - ux0 + vy1 - vy0 + w_hi - w_q;
-                dv /= hx;
-                bq = dt3 * v[4] * dv;
-                P2[6 * NE + tid] = bq;
-                P2[7 * NE + tid] = bp;
-            }
-            if (a >= 1 && a <= nx) {
-                const double h1 = P1[tid + 1], h0 = P1[tid];
-                if (CONS) {
-                    tx_q = tfx * (h1 * ux1 - h0 * ux0);
-                    cx_q = tfx * v[4] * (ux1 - ux0);
-                    P2[3 * NE + tid] = cx_q;
-                } else {
-                    tx_q = tfx * (ux1 + ux0) * (h1 - h0);
+                if (z_general(q)) {
+                    cbox* Bf = fresh(&B);
+                    const int dl = Bf->domlo[2], dh = Bf->domhi[2];
+                    if (ppm_special<PPM>(q, dl, dh, bcl[2], bch[2]))
+                        ppm_edges<PPM, 2>(v, q, dl, dh, bcl[2], bch[2], sm, sp);
                 }
-                P2[tid] = tx_q;
+                const double sig_hi = div_by(dabs(w_hi) * dt, hz);
+                trace_sig(v[4], sm, sp, w_hi, w_q, sig_hi, sig_lo, eps, Ipz, Imz);
+                sig_lo = sig_hi;
+                sz = fz.left ? Ipz_prev : Imz;
+                Ipz_prev = Ipz;
             }
-            if (b >= 1 && b <= ny) {
-                const double h1 = P1[NE + tid + W], h0 = P1[NE + tid];
-                if (CONS) {
-                    ty_q = tfy * (h1 * vy1 - h0 * vy0);
-                    cy_q = tfy * v[4] * (vy1 - vy0);
-                    P2[4 * NE + tid] = cy_q;
-                } else {
-                    ty_q = tfy * (vy1 + vy0) * (h1 - h0);
+            if (GEN) {
+                // boundary stencils of the tile's own faces (another's may
+                // reach past S)
+                const int pI = I - (fx.left ? 1 : 0), pJ = J - (fy.left ? 1 : 0);
+                if (a >= 1 && ppm_special<PPM>(pI, B.domlo[0], B.domhi[0], bcl[0], bch[0]))
+                    sx = predict_special<PPM, 0, 1>(S + si, fx.left, px, gx, I, B.domlo[0],
+                                                    B.domhi[0], bcl[0], bch[0]);
+                if (b >= 1 && ppm_special<PPM>(pJ, B.domlo[1], B.domhi[1], bcl[1], bch[1]))
+                    sy = predict_special<PPM, 1, SW>(S + si, fy.left, py, gy, J, B.domlo[1],
+                                                     B.domhi[1], bcl[1], bch[1]);
+            }
+            if (fx.both | fy.both | fz.both) {  // u == 0 averages the cells
+                if (fx.both && !(dabs(ux) > 0.0)) sx = 0.5 * (S[si - 1] + S[si]);
+                if (fy.both && !(dabs(vy) > 0.0)) sy = 0.5 * (S[si - SW] + S[si]);
+                if (fz.both && !(dabs(w_q) > 0.0)) sz = 0.5 * (v[3] + v[4]);
+            }
+            if (GEN) {
+                if (dx.fixed || dx.clamp)
+                    sx = dx.set(sx, dx.zero ? 0.0 : (dx.lo ? S[si - 1] : S[si]));
+                if (dy.fixed || dy.clamp)
+                    sy = dy.set(sy, dy.zero ? 0.0 : (dy.lo ? S[si - SW] : S[si]));
+            }
+            if (z_general(q)) {
+                const Side dz = side_z(q);
+                if (dz.fixed || dz.clamp) sz = dz.set(sz, dz.zero ? 0.0 : (dz.lo ? v[3] : v[4]));
+            }
+        }
+        HX[tid] = sx;
+        HY[tid] = sy;
+        TZ[tid] = CONS ? tfz * (sz * w_q - sz_p * w_p) : tfz * (w_q + w_p) * (sz - sz_p);
+        double* BBq = lds + oBB + (CONS ? (q & 1) * NT : 0);  // planes q and q - 1
+        double* SCq = lds + oSC + (CONS ? (q & 1) * NT : 0);
+        const double* BBp = lds + oBB + (CONS ? (~q & 1) * NT : 0);
+        double bq = 0.0;
+        if (CONS) {
+            double dv = ULq[ui + 1] - ux + VLq[tid + W] - vy + w_hi - w_q;
+            dv = div_by(dv, hx);
+            bq = dt3 * v[4] * dv;
+            BBq[tid] = bq;
+            SCq[tid] = v[4];
+            CZ[tid] = tfz * v[3] * (w_q - w_p);
+        }
+        __syncthreads();
+
+        // ---- 3: corner-coupled states
+        {
+            const double up = ULp[ui], vp = VLp[tid];  // plane q - 1
+            const Face gx(up, eps, dx.lo, dx.hi), gy(vp, eps, dy.lo, dy.hi);
+            // the transverse y term of the cell at column t and the state s
+            // after it (simhxy); then the same along x (simhyx), and by the z
+            // term of plane q - 1 (simhxz, simhyz)
+            auto ycell = [&](int t, double& tt, double& cc) {
+                const double y1 = VLq[t + W], y0 = VLq[t], h1 = HY[t + W], h0 = HY[t];
+                tt = CONS ? tfy * (h1 * y1 - h0 * y0) : tfy * (y1 + y0) * (h1 - h0);
+                cc = CONS ? tfy * SCq[t] * (y1 - y0) : 0.0;
+            };
+            auto xcell = [&](int t, int u, double& tt, double& cc) {
+                const double x1 = ULq[u + 1], x0 = ULq[u], h1 = HX[t + 1], h0 = HX[t];
+                tt = CONS ? tfx * (h1 * x1 - h0 * x0) : tfx * (x1 + x0) * (h1 - h0);
+                cc = CONS ? tfx * SCq[t] * (x1 - x0) : 0.0;
+            };
+            auto corner_x = [&](double s, int o) {
+                double tt, cc;
+                ycell(tid + o, tt, cc);
+                return CONS ? ((s - tt) - BBq[tid + o]) + cc : s - tt;
+            };
+            auto corner_y = [&](double s, int n) {
+                double tt, cc;
+                xcell(tid + n * W, ui + n * UW, tt, cc);
+                return CONS ? ((s - tt) - BBq[tid + n * W]) + cc : s - tt;
+            };
+            auto corner_z = [&](double s, int t) {
+                return CONS ? ((s - TZ[t]) - BBp[t]) + CZ[t] : s - TZ[t];
+            };
+            double tx_q, ty_q, cx_q, cy_q;
+            ycell(tid, ty_q, cy_q);
+            xcell(tid, ui, tx_q, cx_q);
+            auto corner_f = [&](double s, bool left, double tp, double tq, double cp, double cq) {
+                const double x = s - (left ? tp : tq);
+                return CONS ? (x - (left ? bp : bq)) + (left ? cp : cq) : x;
+            };
+            double xy = corner_x(sx, fx.left ? -1 : 0);
+            double yx = corner_y(sy, fy.left ? -1 : 0);
+            double xz = corner_z(sx_p, tid + (gx.left ? -1 : 0));
+            double yz = corner_z(sy_p, tid + (gy.left ? -W : 0));
+            double zx = corner_f(sz, fz.left, tx_p, tx_q, cx_p, cx_q);
+            double zy = corner_f(sz, fz.left, ty_p, ty_q, cy_p, cy_q);
+            if (fx.both | fy.both | fz.both | gx.both | gy.both) {
+                gcc* sq = s_plane(q);
+                gcc* sp = s_plane(q - 1);
+                if (fx.both)
+                    xy = 0.5 * (corner_x(gload(sq, oCol - 8u), -1) + corner_x(v[4], 0));
+                if (fy.both)
+                    yx = 0.5 * (corner_y(gload(sq, oCol - sjs), -1) + corner_y(v[4], 0));
+                if (gx.both)
+                    xz = 0.5 * (corner_z(gload(sp, oCol - 8u), tid - 1) +
+                                corner_z(v[3], tid));
+                if (gy.both)
+                    yz = 0.5 * (corner_z(gload(sp, oCol - sjs), tid - W) +
+                                corner_z(v[3], tid));
+                if (fz.both) {
+                    zx = 0.5 * (corner_f(v[3], true, tx_p, tx_q, cx_p, cx_q) +
+                                corner_f(v[4], false, tx_p, tx_q, cx_p, cx_q));
+                    zy = 0.5 * (corner_f(v[3], true, ty_p, ty_q, cy_p, cy_q) +
+                                corner_f(v[4], false, ty_p, ty_q, cy_p, cy_q));
                 }
-                P2[NE + tid] = ty_q;
             }
-            if (pplane) {
-                if (CONS) {
-                    P2[2 * NE + tid] = tfz * (hz_q * w_q - hz_p * w_p);
-                    P2[5 * NE + tid] = tfz * v[3] * (w_q - w_p);
-                } else {
-                    P2[2 * NE + tid] = tfz * (w_q + w_p) * (hz_q - hz_p);
-                }
+            if (GEN) {
+                xy = dx.set(xy, sx);
+                yx = dy.set(yx, sy);
+                xz = dx.set(xz, sx_p);
+                yz = dy.set(yz, sy_p);
             }
+            if (z_general(q)) {
+                const Side dz = side_z(q);
+                zx = dz.set(zx, sz);
+                zy = dz.set(zy, sz);
+            }
+            XY[tid] = xy;
+            YX[tid] = yx;
+            XZ[tid] = xz;
+            YZ[tid] = yz;
+            // the z edge terms of plane q - 1
+            EX[tid] = CONS ? efz * (zx * w_q - tzx_p * w_p) : efz * (w_q + w_p) * (zx - tzx_p);
+            EY[tid] = CONS ? efz * (zy * w_q - tzy_p * w_p) : efz * (w_q + w_p) * (zy - tzy_p);
+            FL[tid] = fo_p;
+            tzx_p = zx;
+            tzy_p = zy;
+            tx_p = tx_q;
+            ty_p = ty_q;
+            cx_p = cx_q;
+            cy_p = cy_q;
+            bp = bq;
         }
+        // plane q + 1 takes plane q - 2's slots
+        stage_planes(slot_o);
         __syncthreads();
 
-        // ---- D2: corner-coupled states
-        if (col && a >= 1 && b >= 1 && b <= ny) {  // simhxy, x-faces of plane q
-            double l = apply3<CONS>(slx, P2[NE + tid - 1], CONS ? P2[6 * NE + tid - 1] : 0.0,
-                                    CONS ? P2[4 * NE + tid - 1] : 0.0);
-            double r = apply3<CONS>(srx, P2[NE + tid], CONS ? P2[6 * NE + tid] : 0.0,
-                                    CONS ? P2[4 * NE + tid] : 0.0);
-            if (!XYF) bc_pair(I, dlx, dhx, bcx0, bcx1, vn0, S[si - 1], S[si], l, r);
-            P1[tid] = upwind(l, r, ULq[ui], rel_eps);
-        }
-        if (col && b >= 1 && a >= 1 && a <= nx) {  // simhyx, y-faces of plane q
-            double l = apply3<CONS>(sly, P2[tid - W], CONS ? P2[6 * NE + tid - W] : 0.0,
-                                    CONS ? P2[3 * NE + tid - W] : 0.0);
-            double r = apply3<CONS>(sry, P2[tid], CONS ? P2[6 * NE + tid] : 0.0,
-                                    CONS ? P2[3 * NE + tid] : 0.0);
-            if (!XYF) bc_pair(J, dly, dhy, bcy0, bcy1, vn1, S[si - SW], S[si], l, r);
-            P1[NE + tid] = upwind(l, r, VLq[vi], rel_eps);
-        }
-        if (pplane && col && a >= 1) {  // simhxz, x-faces of plane p
-            double l = apply3<CONS>(slx_p, P2[2 * NE + tid - 1], CONS ? P2[7 * NE + tid - 1] : 0.0,
-                                    CONS ? P2[5 * NE + tid - 1] : 0.0);
-            double r = apply3<CONS>(srx_p, P2[2 * NE + tid], CONS ? P2[7 * NE + tid] : 0.0,
-                                    CONS ? P2[5 * NE + tid] : 0.0);
-            if (!XYF) bc_pair(I, dlx, dhx, bcx0, bcx1, vn0, SC[tid - 1], SC[tid], l, r);
-            P1[2 * NE + tid] = upwind(l, r, ULp[ui], rel_eps);
-        }
-        if (pplane && col && b >= 1) {  // simhyz, y-faces of plane p
-            double l = apply3<CONS>(sly_p, P2[2 * NE + tid - W], CONS ? P2[7 * NE + tid - W] : 0.0,
-                                    CONS ? P2[5 * NE + tid - W] : 0.0);
-            double r = apply3<CONS>(sry_p, P2[2 * NE + tid], CONS ? P2[7 * NE + tid] : 0.0,
-                                    CONS ? P2[5 * NE + tid] : 0.0);
-            if (!XYF) bc_pair(J, dly, dhy, bcy0, bcy1, vn1, SC[tid - W], SC[tid], l, r);
-            P1[3 * NE + tid] = upwind(l, r, VLp[vi], rel_eps);
-        }
-        if (zface && col && a >= 1 && a <= nx) {  // simhzx, z-face q
-            double l = apply3<CONS>(slz, tx_p, bp, cx_p);
-            double r = apply3<CONS>(srz, tx_q, bq, cx_q);
-            bc_pair(q, dlz, dhz, bcz0, bcz1, vn2, v[3], v[4], l, r);
-            tzx_q = upwind(l, r, w_q, rel_eps);
-        }
-        if (zface && col && b >= 1 && b <= ny) {  // simhzy, z-face q
-            double l = apply3<CONS>(slz, ty_p, bp, cy_p);
-            double r = apply3<CONS>(srz, ty_q, bq, cy_q);
-            bc_pair(q, dlz, dhz, bcz0, bcz1, vn2, v[3], v[4], l, r);
-            tzy_q = upwind(l, r, w_q, rel_eps);
-        }
-        __syncthreads();
-
-        // ---- E1: per-cell edge terms
-        if (col && a >= 1 && a <= nx && b >= 1 && b <= ny) {
-            const double ux1 = ULq[ui + 1], ux0 = ULq[ui];
-            const double vy1 = VLq[vi + W], vy0 = VLq[vi];
-            const double t1 = P1[tid + 1], t0 = P1[tid];
-            const double y1 = P1[NE + tid + W], y0 = P1[NE + tid];
-            if (CONS) {
-                exy_q = efx * (t1 * ux1 - t0 * ux0);
-                eyx_q = efy * (y1 * vy1 - y0 * vy0);
-            } else {
-                exy_q = efx * (ux1 + ux0) * (t1 - t0);
-                eyx_q = efy * (vy1 + vy0) * (y1 - y0);
-            }
-        }
-        if (pplane && col) {
-            if (b >= 1 && b <= ny) {
-                const double vy1 = VLp[vi + W], vy0 = VLp[vi];
-                const double t1 = P1[3 * NE + tid + W], t0 = P1[3 * NE + tid];
-                P2[tid] = CONS ? efy * (t1 * vy1 - t0 * vy0) : efy * (vy1 + vy0) * (t1 - t0);
-                P2[NE + tid] = CONS ? efz * (tzy_q * w_q - tzy_p * w_p)
-                                    : efz * (w_q + w_p) * (tzy_q - tzy_p);
-            }
-            if (a >= 1 && a <= nx) {
-                const double ux1 = ULp[ui + 1], ux0 = ULp[ui];
-                const double t1 = P1[2 * NE + tid + 1], t0 = P1[2 * NE + tid];
-                P2[2 * NE + tid] = CONS ? efx * (t1 * ux1 - t0 * ux0) : efx * (ux1 + ux0) * (t1 - t0);
-                P2[3 * NE + tid] = CONS ? efz * (tzx_q * w_q - tzx_p * w_p)
-                                        : efz * (w_q + w_p) * (tzx_q - tzx_p);
-            }
-        }
-        __syncthreads();
-
-        // ---- E2: edge states
-        if (pplane && col && a >= 1 && b >= 1 && b <= ny && (a <= nx || last_x)) {  // x-faces, p
-            double l = slx_p - P2[tid - 1];
-            l = l - P2[NE + tid - 1];
-            double r = srx_p - P2[tid];
-            r = r - P2[NE + tid];
-            const double u0 = ULp[ui];
-            if (CONS) {
-                l = l - dt2hx * SC[tid - 1] * (u0 - ULp[ui - 1]);
-                r = r - dt2hx * SC[tid] * (ULp[ui + 1] - u0);
-            }
-            const double sedgel = l + dt2 * FL[tid - 1];
-            const double sedger = r + dt2 * FL[tid];
-            double res = upwind(sedgel, sedger, u0, rel_eps);
-            if (!XYF)
-                res = bc_edge(res, I, dlx, dhx, bcx0, bcx1, vn0, SC[tid - 1], SC[tid], sedgel,
-                              sedger);
-            e0Col[-e0ks] = res;  // plane p
-            if (flux) flux_store(boxes[bid], 0, I, J, q - 1, comp, flux, u0, res, false);
-        }
-        if (pplane && col && b >= 1 && a >= 1 && a <= nx && (b <= ny || last_y)) {  // y-faces, p
-            double l = sly_p - P2[2 * NE + tid - W];
-            l = l - P2[3 * NE + tid - W];
-            double r = sry_p - P2[2 * NE + tid];
-            r = r - P2[3 * NE + tid];
-            const double u0 = VLp[vi];
-            if (CONS) {
-                l = l - dt2hy * SC[tid - W] * (u0 - VLp[vi - W]);
-                r = r - dt2hy * SC[tid] * (VLp[vi + W] - u0);
-            }
-            const double sedgel = l + dt2 * FL[tid - W];
-            const double sedger = r + dt2 * FL[tid];
-            double res = upwind(sedgel, sedger, u0, rel_eps);
-            if (!XYF)
-                res = bc_edge(res, J, dly, dhy, bcy0, bcy1, vn1, SC[tid - W], SC[tid], sedgel,
-                              sedger);
-            e1Col[-e1ks] = res;  // plane p
-            if (flux) flux_store(boxes[bid], 1, I, J, q - 1, comp, flux, u0, res, false);
-        }
-        if (((zface && q <= z1) || (q == z1 + 1 && last_z)) && col && a >= 1 && a <= nx &&
-            b >= 1 && b <= ny) {  // z-face q
-            double l = slz - exy_p;
-            l = l - eyx_p;
-            double r = srz - exy_q;
-            r = r - eyx_q;
-            if (CONS) {
-                l = l - dt2hz * v[3] * (w_q - w_p);
-                r = r - dt2hz * v[4] * (w_hi - w_q);
-            }
-            const double sedgel = l + dt2 * fo_p;
-            const double sedger = r + dt2 * fo_q;
-            double res = upwind(sedgel, sedger, w_q, rel_eps);
-            res = bc_edge(res, q, dlz, dhz, bcz0, bcz1, vn2, v[3], v[4], sedgel, sedger);
-            *e2Col = res;  // z-face q
-            if (flux) flux_store(boxes[bid], 2, I, J, q, comp, flux, w_q, res, true);
-        }
-
-        // ---- advance the column state to the next plane
-        slx_p = slx;
-        srx_p = srx;
-        sly_p = sly;
-        sry_p = sry;
-        hz_p = hz_q;
-        tx_p = tx_q;
-        ty_p = ty_q;
-        cx_p = cx_q;
-        cy_p = cy_q;
-        bp = bq;
-        tzx_p = tzx_q;
-        tzy_p = tzy_q;
-        exy_p = exy_q;
-        eyx_p = eyx_q;
-        w_p = w_q;
-        w_q = w_hi;
-        fo_p = fo_q;
-        wCol += wks;
-        e0Col += e0ks;
-        e1Col += e1ks;
-        e2Col += e2ks;
+        advance(q < z1);
+        const int s_new = slot_o;
+        slot_o = slot_p;
         slot_p = slot_q;
-        slot_q = slot_q == 2 ? 0 : slot_q + 1;
+        slot_q = s_new;
     }
+    edges(z1 + 2);
 }
 
 }  // namespace
@@ -779,6 +844,19 @@ bool fused_edge_scal_ok(const mx_adv_ctx* c, int is_conservative) {
            c->p.ppm_trace_forces == 0 && c->fused_edge;
 }
 
+// a tile and its stencil span at most 25 rows (32-bit byte offsets in a plane)
+bool fused_edge_rows_ok(const EdgeLevel& L) {
+    const long long lim = 0x7fffffffLL / (8 * 26);
+    auto ok = [&](const mx_multifab* m) {
+        for (int b = 0; b < m->nfab; ++b)
+            if (m->fab[b].jstride > lim) return false;
+        return true;
+    };
+    bool r = ok(L.state) && ok(L.force);
+    for (int d = 0; d < 3; ++d) r = r && ok(&L.umac->dir[d]) && ok(&L.sedge->dir[d]);
+    return r;
+}
+
 namespace {
 
 // does boundary code `bc` override anything (everything but INT_DIR)?
@@ -787,20 +865,26 @@ bool bc_acts(int bc) {
            bc == MX_BC_REFLECT_EVEN || bc == MX_BC_REFLECT_ODD;
 }
 
-// A tile is x/y-free when, in x and in y, each domain side either carries no
-// override for any component or lies beyond the tile's reach: the kernel
-// evaluates cells [X0 - 1, X0 + nx] (PPM boundary stencils act within three
-// cells of a side) and faces [X0, X0 + nx] (face overrides act on the side's
-// face).
-bool tile_xy_free(const int lo0, int n, int dlo, int dhi, bool act_lo, bool act_hi) {
-    const bool free_lo = !act_lo || lo0 - 1 > dlo + 2;
-    const bool free_hi = !act_hi || lo0 + n < dhi - 2;
-    return free_lo && free_hi;
+// does it do more than pick the inside cell's state on the side's face?
+// (hoextrap has PPM boundary stencils; extrapolation clamps a normal velocity)
+bool bc_general(int bc, int is_vel) {
+    return bc_acts(bc) && bc != MX_BC_REFLECT_EVEN && (bc != MX_BC_FOEXTRAP || is_vel);
 }
 
-template <int TX, int TY, int WPE, bool XYF>
+// A tile's chunk is out of reach of a direction's sides when each either
+// carries no such condition for any component or lies beyond it: the kernel
+// evaluates cells [lo0 - 1, lo0 + n] (PPM boundary stencils act within three
+// cells of a side) and faces [lo0, lo0 + n] (face overrides act on the side's
+// face).
+bool tile_clear(const int lo0, int n, int dlo, int dhi, bool act_lo, bool act_hi) {
+    const bool clear_lo = !act_lo || lo0 - 1 > dlo + 2;
+    const bool clear_hi = !act_hi || lo0 + n < dhi - 2;
+    return clear_lo && clear_hi;
+}
+
+template <int TX, int TY, int MODE>
 int launch_one(mx_adv_ctx* c, const FBox* db, const FTile* dtl, size_t ntile, const FComp* dc,
-               const KGeom& kg, const FArgs& A, int num_comp, bool cons) {
+               const FArgs& A, int num_comp, bool cons) {
     if (ntile == 0) return MX_OK;
     const int xm = c->es_fused_xcd;
     const dim3 grid = xm ? dim3(xcd_tile_blocks((long long)ntile, num_comp))
@@ -809,32 +893,34 @@ int launch_one(mx_adv_ctx* c, const FBox* db, const FTile* dtl, size_t ntile, co
     dim3 block(fused_nt(TX, TY));
     if (c->p.ppm_type == 1) {
         if (cons)
-            MX_LAUNCH(c, "k_es_fused", (k_es_fused<1, true, TX, TY, XYF, WPE>), grid, block, db, dtl, dc, kg, A, nt, xm);
+            MX_LAUNCH(c, "k_es_fused", (k_es_fused<1, true, TX, TY, MODE>), grid, block, db, dtl, dc, A, nt, xm);
         else
-            MX_LAUNCH(c, "k_es_fused", (k_es_fused<1, false, TX, TY, XYF, WPE>), grid, block, db, dtl, dc, kg, A, nt, xm);
+            MX_LAUNCH(c, "k_es_fused", (k_es_fused<1, false, TX, TY, MODE>), grid, block, db, dtl, dc, A, nt, xm);
     } else {
         if (cons)
-            MX_LAUNCH(c, "k_es_fused", (k_es_fused<2, true, TX, TY, XYF, WPE>), grid, block, db, dtl, dc, kg, A, nt, xm);
+            MX_LAUNCH(c, "k_es_fused", (k_es_fused<2, true, TX, TY, MODE>), grid, block, db, dtl, dc, A, nt, xm);
         else
-            MX_LAUNCH(c, "k_es_fused", (k_es_fused<2, false, TX, TY, XYF, WPE>), grid, block, db, dtl, dc, kg, A, nt, xm);
+            MX_LAUNCH(c, "k_es_fused", (k_es_fused<2, false, TX, TY, MODE>), grid, block, db, dtl, dc, A, nt, xm);
     }
     return MX_OK;
 }
 
-template <int TX, int TY, int WPE>
+template <int TX, int TY>
 int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int is_vel,
                  const mx_bcrec* bcs, const std::vector<int>& scomps,
                  const std::vector<int>& bccomps, int is_conservative) {
     const int num_comp = (int)scomps.size();
-    const long long lim = 0x7fffffffLL;
     std::vector<FBox> boxes;
-    std::vector<FTile> tiles, btiles;  // x/y-free tiles, then the others
-    bool act[2][2] = {{false, false}, {false, false}};
+    bool zgen = false;
+    std::vector<FTile> tiles, btiles;  // tiles clear of general x/y sides, then the others
+    bool act[3][2] = {{false, false}, {false, false}, {false, false}};
     for (int vc = 0; vc < num_comp; ++vc)
-        for (int d = 0; d < 2; ++d) {
-            act[d][0] = act[d][0] || bc_acts(bcs[bccomps[vc]].lo[d]);
-            act[d][1] = act[d][1] || bc_acts(bcs[bccomps[vc]].hi[d]);
+        for (int d = 0; d < 3; ++d) {
+            act[d][0] = act[d][0] || bc_general(bcs[bccomps[vc]].lo[d], is_vel);
+            act[d][1] = act[d][1] || bc_general(bcs[bccomps[vc]].hi[d], is_vel);
         }
+    const double dt = c->p.dt, dt2 = 0.5 * dt, dt3 = dt / 3.0, dt4 = 0.25 * dt, dt6 = dt / 6.0;
+    const bool cons = is_conservative != 0;
     for (const EdgeLevel& L : levs) {
         const auto& grids = c->grids[L.lev];
         for (size_t b = 0; b < grids.size(); ++b) {
@@ -842,9 +928,8 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
             FBox B;
             HBox g = hbox(grids[b]);
             for (int q = 0; q < 3; ++q) {
-                B.lo[q] = g.lo[q];
                 B.hi[q] = g.hi[q];
-                B.dx[q] = c->p.dx[L.lev][q];
+                B.h[q] = div_const(c->p.dx[L.lev][q]);
                 B.domlo[q] = c->p.domain_lo[L.lev][q];
                 B.domhi[q] = c->p.domain_hi[L.lev][q];
             }
@@ -859,25 +944,32 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
             B.bc_b = L.bc_b;
             B.be_a = L.be_a;
             B.be_b = L.be_b;
-            // the kernel keeps the plane strides in 32 bits
-            const DA* views[] = {&B.s,     &B.fo,    &B.um[0], &B.um[1],
-                                 &B.um[2], &B.se[0], &B.se[1], &B.se[2]};
-            for (const DA* d : views)
-                if (d->js > lim || d->ks > lim) return MX_ERR_UNSUPPORTED;
-            const int ntx = (g.hi[0] - g.lo[0] + TX) / TX;
-            const int nty = (g.hi[1] - g.lo[1] + TY) / TY;
-            const int nzc = (g.hi[2] - g.lo[2] + tz) / tz;
+            const DA* strided[] = {&B.s,     &B.fo,    &B.um[0], &B.um[1],
+                                   &B.um[2], &B.se[0], &B.se[1], &B.se[2]};
+            for (int q = 0; q < 8; ++q) B.ks[q] = 8 * strided[q]->ks;
             const int id = (int)boxes.size();
-            for (int z = 0; z < nzc; ++z)
-                for (int y = 0; y < nty; ++y)
-                    for (int x = 0; x < ntx; ++x) {
-                        const int x0 = g.lo[0] + x * TX, y0 = g.lo[1] + y * TY;
-                        const int nx = std::min(TX, g.hi[0] - x0 + 1);
-                        const int ny = std::min(TY, g.hi[1] - y0 + 1);
-                        const bool f =
-                            tile_xy_free(x0, nx, B.domlo[0], B.domhi[0], act[0][0], act[0][1]) &&
-                            tile_xy_free(y0, ny, B.domlo[1], B.domhi[1], act[1][0], act[1][1]);
-                        (f ? tiles : btiles).push_back({id, x, y, z});
+            for (int z = g.lo[2]; z <= g.hi[2]; z += tz)
+                for (int y = g.lo[1]; y <= g.hi[1]; y += TY)
+                    for (int x = g.lo[0]; x <= g.hi[0]; x += TX) {
+                        FTile T{id,
+                                x,
+                                y,
+                                z,
+                                std::min(TX, g.hi[0] - x + 1),
+                                std::min(TY, g.hi[1] - y + 1),
+                                std::min(tz, g.hi[2] - z + 1),
+                                0};
+                        const int t0[3] = {x, y, z}, tn[3] = {T.nx, T.ny, T.nz};
+                        bool f = true;
+                        for (int d = 0; d < 2; ++d)
+                            f = f && tile_clear(t0[d], tn[d], B.domlo[d], B.domhi[d], act[d][0],
+                                                act[d][1]);
+                        for (int s = 0; s < 2; ++s)
+                            if (!tile_clear(z, T.nz, B.domlo[2], B.domhi[2], s == 0 && act[2][0],
+                                            s == 1 && act[2][1]))
+                                T.zgen |= 1 << s;
+                        (f ? tiles : btiles).push_back(T);
+                        zgen = zgen || (f && T.zgen);
                     }
             boxes.push_back(B);
         }
@@ -895,11 +987,8 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
         comps[vc].comp = scomps[vc];
         comps[vc].flux = (levs[0].sflux && scomps[vc] == levs[0].flux_comp) ? levs[0].flux_kind : 0;
     }
-    FArgs A;
-    A.start_scomp = scomps[0];
-    A.num_comp = num_comp;
-    A.is_vel = is_vel;
-    A.tz = tz;
+    const FArgs A{dt,     c->p.rel_eps,      dt2,      dt3, cons ? dt3 : dt6, cons ? dt2 : dt4,
+                  num_comp, is_vel};
     Table tab(c);
     size_t ob = tab.add(boxes);
     size_t ot = tab.add(tiles);
@@ -909,24 +998,22 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
     const FBox* db = tab.dev<FBox>(ob);
     const FTile* dtl = tab.dev<FTile>(ot);
     const FComp* dc = tab.dev<FComp>(oc);
-    KGeom kg = kgeom(c, levs[0].lev);
-    const bool cons = is_conservative != 0;
-    rc = launch_one<TX, TY, WPE, true>(c, db, dtl, nfree, dc, kg, A, num_comp, cons);
+    // a z side that needs more than the upwind cell puts every clear tile in the
+    // kernel with the z rules (3 waves per SIMD): apart, the chunks at the side
+    // and the others would each leave the chip half empty
+    rc = zgen ? launch_one<TX, TY, 1>(c, db, dtl, nfree, dc, A, num_comp, cons)
+              : launch_one<TX, TY, 0>(c, db, dtl, nfree, dc, A, num_comp, cons);
     if (rc) return rc;
-    return launch_one<TX, TY, WPE, false>(c, db, dtl + nfree, tiles.size() - nfree, dc, kg, A,
-                                     num_comp, cons);
+    return launch_one<TX, TY, 2>(c, db, dtl + nfree, tiles.size() - nfree, dc, A, num_comp, cons);
 }
 
 // the tile shape of `fused_tile`, with the block size (columns rounded up to
 // whole waves) and the register budget (waves per SIMD):
 //   0: 32 x 8 (384 threads), 1: 16 x 16 (384), 2: 16 x 12 (256), 3: 16 x 8 (192),
 //   4: 16 x 11 (256)
-// all at 3 waves per SIMD (168 VGPRs), so a CU holds 2, 2, 3, 4 or 3 blocks.
-// -1 (the default) is 16 x 11: with ppm_type 1 its face phases (19 x 13
-// x-faces, 18 x 14 y-faces) fit one pass of 256 threads, where 16 x 12
-// leaves one wave a second pass while the others wait at the barrier; with
-// ppm_type 2 its x/y-free variant spills 1 VGPR against 7 for 16 x 12
-// (5.50 against 5.57 ms per 256^3 pass)
+// -1 (the default) is 16 x 11: with ppm_type 1 its face values (19 x 13
+// x-faces, 18 x 14 y-faces) are one item per thread of 256, and its LDS is the
+// largest of which a CU holds four blocks
 int fused_tile_of(const mx_adv_ctx* c) {
     if (c->fused_tile >= 0) return c->fused_tile;
     return 4;
@@ -935,11 +1022,11 @@ int launch_tile(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int i
                 const mx_bcrec* bcs, const std::vector<int>& sc, const std::vector<int>& bc,
                 int cons) {
     switch (fused_tile_of(c)) {
-        case 1: return launch_fused<16, 16, 3>(c, levs, tz, is_vel, bcs, sc, bc, cons);
-        case 2: return launch_fused<16, 12, 3>(c, levs, tz, is_vel, bcs, sc, bc, cons);
-        case 3: return launch_fused<16, 8, 3>(c, levs, tz, is_vel, bcs, sc, bc, cons);
-        case 4: return launch_fused<16, 11, 3>(c, levs, tz, is_vel, bcs, sc, bc, cons);
-        default: return launch_fused<32, 8, 3>(c, levs, tz, is_vel, bcs, sc, bc, cons);
+        case 1: return launch_fused<16, 16>(c, levs, tz, is_vel, bcs, sc, bc, cons);
+        case 2: return launch_fused<16, 12>(c, levs, tz, is_vel, bcs, sc, bc, cons);
+        case 3: return launch_fused<16, 8>(c, levs, tz, is_vel, bcs, sc, bc, cons);
+        case 4: return launch_fused<16, 11>(c, levs, tz, is_vel, bcs, sc, bc, cons);
+        default: return launch_fused<32, 8>(c, levs, tz, is_vel, bcs, sc, bc, cons);
     }
 }
 

@@ -132,7 +132,7 @@ struct mx_adv_ctx {
                                  // fused edge kernel's epilogue
     int vp_fused_tile = 2; // its tile (waves per SIMD): 0 16x11 (3), 1 16x8 (3), 2 16x11 (4), 3 32x8 (3)
     int fused_tile = -1;    // 0: 32 x 8 columns, 1: 16 x 16, 2: 16 x 12, 3: 16 x 8,
-                            // 4: 16 x 11; -1: 16 x 11 for ppm_type 1, else 16 x 12
+                            // 4: 16 x 11; -1: 16 x 11
     int fused_per_box = 0;  // 1: one fused launch per box (comparison mode)
     int adj_state_fused = 1;  // adjoint: face, slope and state adjoints in one gather
     int adj_face_sums = 0;    // adjoint: predictor-state face adjoints stored once per face
@@ -431,6 +431,8 @@ struct EdgeLevel {
     const double *bc_a = nullptr, *bc_b = nullptr, *be_a = nullptr, *be_b = nullptr;
 };
 bool fused_edge_scal_ok(const mx_adv_ctx* c, int is_conservative);
+// do the rows of the level's FABs fit the kernel's 32-bit byte offsets?
+bool fused_edge_rows_ok(const EdgeLevel& L);
 int make_edge_scal_fused_levels(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int is_vel,
                                 const mx_bcrec* bcs, int start_scomp, int start_bccomp,
                                 int num_comp, int is_conservative);

@@ -636,7 +636,8 @@ int make_edge_scal(mx_adv_ctx* c, int lev, const mx_multifab* state,
                    const mx_multifab* force, int is_vel, const mx_bcrec* bcs, int nbccomp,
                    int start_scomp, int start_bccomp, int num_comp, int is_conservative) {
     (void)nbccomp;
-    if (fused_edge_scal_ok(c, is_conservative))
+    if (fused_edge_scal_ok(c, is_conservative) &&
+        fused_edge_rows_ok({lev, state, sedge, umac, force}))
         return make_edge_scal_fused(c, lev, state, sedge, umac, force, is_vel, bcs, start_scomp,
                                     start_bccomp, num_comp, is_conservative);
     const int dim = c->p.dim;
@@ -1020,9 +1021,13 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
     // as the fused edge kernel's epilogue (the flux from the edge state in
     // registers); the register updates of reflux_type 2 follow as usual
     const int ept = p.enthalpy_pred_type;
-    const bool rhoh_epilogue = fused_edge_scal_ok(c, 0) && c->rhoh_flux_epilogue && !sph &&
-                               (ept == 0 || ept == 1 || ept == 3);
-    if (fused_edge_scal_ok(c, 0)) {
+    bool fused = fused_edge_scal_ok(c, 0);
+    for (int i = 0; i < nlev; ++i)
+        fused = fused && fused_edge_rows_ok({lev0 + i, &a[i].scal, &a[i].sedge, &a[i].umac,
+                                             &a[i].scal_force});
+    const bool rhoh_epilogue =
+        fused && c->rhoh_flux_epilogue && !sph && (ept == 0 || ept == 1 || ept == 3);
+    if (fused) {
         std::vector<EdgeLevel> levs;
         for (int i = 0; i < nlev; ++i) {
             EdgeLevel L{lev0 + i, &a[i].scal, &a[i].sedge, &a[i].umac, &a[i].scal_force};
