@@ -193,7 +193,10 @@ int mx_adv_prof_read(mx_adv_ctx* ctx, int idx, const char** name, double* total_
                         no traced forces runs as one z-marching kernel;
                         0: the three-kernel form (PPM, transverse, edges),
                         which also serves ppm_type 0, traced forces and 2-D.
-     "edge_scal_tz"     planes per z-chunk of the fused kernel (default 32).
+     "edge_scal_tz"     planes per z-chunk of the fused kernel (1-4096); unset,
+                        the launch picks it from its boxes, so that short
+                        chunks fill the chip and long ones save lead-in
+                        planes; a box is cut into equal chunks.
      "edge_scal_tile"   cell columns per block of the fused kernel, and the
                         block size: 0: 32 x 8 (384 threads), 1: 16 x 16 (384),
                         2: 16 x 12 (256), 3: 16 x 8 (192), 4: 16 x 11 (256);

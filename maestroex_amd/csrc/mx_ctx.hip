@@ -2,6 +2,7 @@
 // fill (FillBoundary + FillUmacGhost), Addw0, CelltoEdge and the unit-level
 // PPM / slope entry points of libmaestroex_amd.so.
 #include <algorithm>
+#include <cmath>
 #include <array>
 #include <cstdio>
 
@@ -10,6 +11,47 @@
 using namespace mxd;
 
 namespace mxh {
+
+// The z-marching kernels' chunk length for a launch.  A block takes about 5
+// steps more than its planes (two planes whose states its first and last faces
+// need, its tables and first loads, its last edges).  A CU steps its resident
+// blocks together: n of the most it holds take a step in (0.86 + 0.14 n / most)
+// of the time of all of them (the edge kernel: 4.3 us alone, 4.8 us with 4).
+// Blocks past a full chip's take another round, and the rounds of a long
+// launch end raggedly (a quarter of a block).  So short chunks fill an idle
+// chip and even out the last round, and cost lead-in planes where there is work
+// for many rounds.  The edge kernel against chunks of 32 planes everywhere: one
+// 32^3 box 0.161 -> 0.031 ms (30 -> 480 blocks), 50^3 in 8 boxes 0.094 -> 0.051
+// ms, 256^3 unchanged; the best chunk of a sweep is 0 to 3% faster.
+int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, int blocks_per_cu) {
+    constexpr int kCus = 256;
+    const double slots = (double)kCus * blocks_per_cu;
+    static const int cand[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64};
+    int best = 32;
+    double best_t = 1e300;
+    for (int tz : cand) {
+        double nb = 0.0, steps = 0.0;
+        int lmax = 0;
+        for (const ChunkCols& c : cols) {
+            const int n = chunk_count(c.nz, tz);
+            const double w = (double)c.tiles * nvar;
+            nb += w * n;
+            steps += w * (c.nz + 5.0 * n);
+            lmax = std::max(lmax, (c.nz + n - 1) / n + 5);
+        }
+        if (nb <= 0.0) break;
+        const double full = std::floor(nb / slots);
+        const double rem = std::ceil((nb - full * slots) / kCus);
+        const double last = rem > 0.0 ? 0.86 + 0.14 * rem / blocks_per_cu : 0.0;
+        const double t = full > 0.0 ? (full + last) * steps / nb + 0.25 * lmax : last * lmax;
+        if (t < best_t * 0.995) {
+            best_t = t;
+            best = tz;
+        }
+    }
+    return best;
+}
+
 
 KGeom kgeom(const mx_adv_ctx* c, int lev) {
     KGeom g;

@@ -905,6 +905,21 @@ int launch_one(mx_adv_ctx* c, const FBox* db, const FTile* dtl, size_t ntile, co
     return MX_OK;
 }
 
+// blocks of the open-boundary kernel a CU holds
+template <int PPM, bool CONS, int TX, int TY>
+int fused_blocks() {
+    static const int n = [] {
+        int v = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_es_fused<PPM, CONS, TX, TY, 0>,
+                                                         fused_nt(TX, TY), 0) != hipSuccess) {
+            (void)hipGetLastError();
+            v = 0;
+        }
+        return v > 0 ? v : 3;
+    }();
+    return n;
+}
+
 template <int TX, int TY>
 int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int is_vel,
                  const mx_bcrec* bcs, const std::vector<int>& scomps,
@@ -912,6 +927,8 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
     const int num_comp = (int)scomps.size();
     std::vector<FBox> boxes;
     bool zgen = false;
+    std::vector<HBox> hb;
+    std::vector<ChunkCols> cols;
     std::vector<FTile> tiles, btiles;  // tiles clear of general x/y sides, then the others
     bool act[3][2] = {{false, false}, {false, false}, {false, false}};
     for (int vc = 0; vc < num_comp; ++vc)
@@ -947,32 +964,46 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
             const DA* strided[] = {&B.s,     &B.fo,    &B.um[0], &B.um[1],
                                    &B.um[2], &B.se[0], &B.se[1], &B.se[2]};
             for (int q = 0; q < 8; ++q) B.ks[q] = 8 * strided[q]->ks;
-            const int id = (int)boxes.size();
-            for (int z = g.lo[2]; z <= g.hi[2]; z += tz)
-                for (int y = g.lo[1]; y <= g.hi[1]; y += TY)
-                    for (int x = g.lo[0]; x <= g.hi[0]; x += TX) {
-                        FTile T{id,
-                                x,
-                                y,
-                                z,
-                                std::min(TX, g.hi[0] - x + 1),
-                                std::min(TY, g.hi[1] - y + 1),
-                                std::min(tz, g.hi[2] - z + 1),
-                                0};
-                        const int t0[3] = {x, y, z}, tn[3] = {T.nx, T.ny, T.nz};
-                        bool f = true;
-                        for (int d = 0; d < 2; ++d)
-                            f = f && tile_clear(t0[d], tn[d], B.domlo[d], B.domhi[d], act[d][0],
-                                                act[d][1]);
-                        for (int s = 0; s < 2; ++s)
-                            if (!tile_clear(z, T.nz, B.domlo[2], B.domhi[2], s == 0 && act[2][0],
-                                            s == 1 && act[2][1]))
-                                T.zgen |= 1 << s;
-                        (f ? tiles : btiles).push_back(T);
-                        zgen = zgen || (f && T.zgen);
-                    }
             boxes.push_back(B);
+            hb.push_back(g);
+            cols.push_back({g.hi[2] - g.lo[2] + 1, (long long)((g.hi[0] - g.lo[0] + TX) / TX) *
+                                                       ((g.hi[1] - g.lo[1] + TY) / TY)});
         }
+    }
+    if (tz <= 0) {
+        const int per_cu = c->p.ppm_type == 1
+                               ? (cons ? fused_blocks<1, true, TX, TY>() : fused_blocks<1, false, TX, TY>())
+                               : (cons ? fused_blocks<2, true, TX, TY>() : fused_blocks<2, false, TX, TY>());
+        tz = pick_chunks(cols, num_comp, per_cu);
+    }
+    for (size_t id = 0; id < boxes.size(); ++id) {
+        const HBox& g = hb[id];
+        const FBox& B = boxes[id];
+        const int nz = g.hi[2] - g.lo[2] + 1, nch = chunk_count(nz, tz);
+        for (int ch = 0; ch < nch; ++ch)
+            for (int y = g.lo[1]; y <= g.hi[1]; y += TY)
+                for (int x = g.lo[0]; x <= g.hi[0]; x += TX) {
+                    const int z = chunk_start(nz, nch, ch), ze = chunk_start(nz, nch, ch + 1);
+                    FTile T{(int)id,
+                            x,
+                            y,
+                            g.lo[2] + z,
+                            std::min(TX, g.hi[0] - x + 1),
+                            std::min(TY, g.hi[1] - y + 1),
+                            ze - z,
+                            0};
+                    const int t0[2] = {x, y}, tn[2] = {T.nx, T.ny};
+                    bool f = true;
+                    for (int d = 0; d < 2; ++d)
+                        f = f && tile_clear(t0[d], tn[d], B.domlo[d], B.domhi[d], act[d][0],
+                                            act[d][1]);
+                    for (int s = 0; s < 2; ++s)
+                        if (!tile_clear(T.z0, T.nz, B.domlo[2], B.domhi[2], s == 0 && act[2][0],
+                                        s == 1 && act[2][1]))
+                            T.zgen |= 1 << s;
+                    (f ? tiles : btiles).push_back(T);
+                    zgen = zgen || (f && T.zgen);
+                }
     }
     const size_t nfree = tiles.size();
     tiles.insert(tiles.end(), btiles.begin(), btiles.end());
@@ -1037,7 +1068,7 @@ int make_edge_scal_fused_list(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs,
                               const std::vector<int>& bccomps, int is_conservative) {
     if (levs.empty() || scomps.empty()) return MX_OK;
     if (scomps.size() != bccomps.size()) return MX_ERR_ARG;
-    const int tz = c->fused_tz > 0 ? c->fused_tz : 32;
+    const int tz = c->fused_tz;
     if (c->fused_per_box) {
         // comparison mode: the same work as one launch per box
         std::vector<EdgeLevel> one(1);

@@ -116,7 +116,7 @@ struct mx_adv_ctx {
 
     // kernel selection (mx_adv_set_tuning)
     int fused_edge = 1;
-    int fused_tz = 32;
+    int fused_tz = 0;  // planes per z-chunk of the fused edge kernel; 0: pick_chunks
     int vp_fused_xcd = -1; // fused VelPred: XCD-aware block order (xcd_tile mode); -1: 2 for
                            // one level of equal boxes, else 1
     int es_fused_xcd = 1;  // fused MakeEdgeScal: XCD-aware block order (xcd_tile mode)
@@ -323,6 +323,21 @@ struct Table {
         return reinterpret_cast<const T*>(base + off);
     }
 };
+
+// The z-marching kernels' chunks.  A level's tile columns by box: `tiles` columns
+// of `nz` planes; `nvar` blocks (components) per column chunk.
+struct ChunkCols {
+    int nz;
+    long long tiles;
+};
+// the number of chunks a box of nz planes is cut into for chunks of about tz, and
+// where chunk i of n starts: equal chunks, the longer ones first
+inline int chunk_count(int nz, int tz) { return (nz + tz - 1) / tz; }
+inline int chunk_start(int nz, int n, int i) {
+    const int q = nz / n, r = nz % n;
+    return i * q + (i < r ? i : r);
+}
+int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, int blocks_per_cu);
 
 // launch geometry: x covers the largest per-box region, y = boxes, z = extra
 inline dim3 grid_for(long long maxpts, int nbox, int nz, int block) {
