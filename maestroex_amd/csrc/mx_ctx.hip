@@ -23,27 +23,31 @@ namespace mxh {
 // for many rounds.  The edge kernel against chunks of 32 planes everywhere: one
 // 32^3 box 0.161 -> 0.031 ms (30 -> 480 blocks), 50^3 in 8 boxes 0.094 -> 0.051
 // ms, 256^3 unchanged; the best chunk of a sweep is 0 to 3% faster.
-int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, int blocks_per_cu) {
+int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, const int blocks_per_cu[2]) {
     constexpr int kCus = 256;
-    const double slots = (double)kCus * blocks_per_cu;
     static const int cand[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64};
     int best = 32;
     double best_t = 1e300;
     for (int tz : cand) {
-        double nb = 0.0, steps = 0.0;
-        int lmax = 0;
-        for (const ChunkCols& c : cols) {
-            const int n = chunk_count(c.nz, tz);
-            const double w = (double)c.tiles * nvar;
-            nb += w * n;
-            steps += w * (c.nz + 5.0 * n);
-            lmax = std::max(lmax, (c.nz + n - 1) / n + 5);
+        double t = 0.0;
+        for (int l = 0; l < 2; ++l) {
+            double nb = 0.0, steps = 0.0;
+            int lmax = 0;
+            for (const ChunkCols& c : cols) {
+                if (!c.tiles[l]) continue;
+                const int n = chunk_count(c.nz, tz);
+                const double w = (double)c.tiles[l] * nvar;
+                nb += w * n;
+                steps += w * (c.nz + 5.0 * n);
+                lmax = std::max(lmax, (c.nz + n - 1) / n + 5);
+            }
+            if (nb <= 0.0) continue;
+            const double slots = (double)kCus * blocks_per_cu[l];
+            const double full = std::floor(nb / slots);
+            const double rem = std::ceil((nb - full * slots) / kCus);
+            const double last = rem > 0.0 ? 0.86 + 0.14 * rem / blocks_per_cu[l] : 0.0;
+            t += full > 0.0 ? (full + last) * steps / nb + 0.25 * lmax : last * lmax;
         }
-        if (nb <= 0.0) break;
-        const double full = std::floor(nb / slots);
-        const double rem = std::ceil((nb - full * slots) / kCus);
-        const double last = rem > 0.0 ? 0.86 + 0.14 * rem / blocks_per_cu : 0.0;
-        const double t = full > 0.0 ? (full + last) * steps / nb + 0.25 * lmax : last * lmax;
         if (t < best_t * 0.995) {
             best_t = t;
             best = tz;

@@ -51,14 +51,12 @@
 #include <climits>
 
 #include "mx_internal.H"
+#include "mx_march.H"
 
 using namespace mxd;
 using namespace mxh;
 
 namespace {
-
-typedef __attribute__((address_space(1))) const double gcd;
-typedef __attribute__((address_space(1))) double gd;
 
 // threads of a block: the tile's columns grown by one cell on each side,
 // rounded up to whole waves
@@ -109,21 +107,6 @@ struct FArgs {
     int num_comp;
     int is_vel;
 };
-
-typedef __attribute__((address_space(1))) const char gcc;
-typedef __attribute__((address_space(1))) char gc;
-
-// a double at a uniform base plus a 32-bit byte offset.  The empty asm keeps
-// the offset's widening beside the access, where the compiler folds it into
-// the addressing mode (one VGPR per address, no 64-bit add).
-__device__ __forceinline__ double gload(gcc* base, unsigned off) {
-    asm("" : "+v"(off));
-    return *(gcd*)(base + off);
-}
-__device__ __forceinline__ void gstore(gc* base, unsigned off, double v) {
-    asm("" : "+v"(off));
-    *(gd*)(base + off) = v;
-}
 
 // The table's pointer, behind the optimiser's back: what is read from it is
 // read (by scalar loads, from the constant address space) where it is used, not
@@ -199,66 +182,6 @@ struct Face {
         traced = off & !(left ^ up);
     }
 };
-
-// trace of the upwind cell to its face (ppm_trace of mx_device.H for one
-// side): A the edge value at the face, B the cell's other edge value.
-// sp - h (sp - sm - c s6) and sm + h (sp - sm + c s6) are both
-// A + h ((B - A) + c s6).
-__device__ __forceinline__ double trace_face(double s0, double A, double B, double sig) {
-    // 3 x and 6 x rounded once, by inline constants: 2 x + x, twice that
-    const double s3 = fma(2.0, s0, s0), ab = A + B;
-    const double s6 = 2.0 * s3 - fma(2.0, ab, ab);
-    return A + 0.5 * sig * ((B - A) + (1.0 - 2.0 / 3.0 * sig) * s6);
-}
-
-// the CW84 limiter (cw_limit of mx_device.H, symmetric in its two edges)
-// and the trace
-__device__ __forceinline__ double cw_trace(double s0, double A, double B, double sig) {
-    const double a = A - s0, b = s0 - B;
-    const bool flat = a * b <= 0.0;
-    const bool ca = dabs(a) >= 2.0 * dabs(b);
-    const bool cb = dabs(b) >= 2.0 * dabs(a);
-    const double s3 = fma(2.0, s0, s0);  // 3 s0
-    const double A2 = s3 - 2.0 * B, B2 = s3 - 2.0 * A;
-    const double A1 = ca ? A2 : A;
-    const double B1 = (cb && !ca) ? B2 : B;
-    return trace_face(s0, flat ? s0 : A1, flat ? s0 : B1, sig);
-}
-
-// The predictor's upwind state on the low face of a cell along a direction, s
-// the cell's S slot and F its low face value's (FST, SST: one cell along the
-// direction in the face and the S plane).
-template <int PPM, int FST, int SST>
-__device__ __forceinline__ double predict(const double* s, const double* F, bool left, bool traced,
-                                          double sig) {
-    const double* c = s + (left ? -SST : 0);
-    const double s0 = c[0];
-    double x;
-    if (PPM == 1) {
-        x = cw_trace(s0, F[0], F[left ? -FST : FST], sig);
-    } else {
-        const double* Fc = F + (left ? -FST : 0);
-        double w9[9], sm, sp;
-#pragma unroll
-        for (int o = -4; o <= 4; ++o) w9[4 + o] = (o >= -2 && o <= 2) ? c[o * SST] : 0.0;
-        cs_cell(w9, Fc[-FST], Fc[0], Fc[FST], Fc[2 * FST], 1.e-10, sm, sp);
-        x = trace_face(s0, left ? sp : sm, left ? sm : sp, sig);
-    }
-    return traced ? x : s0;
-}
-// the same with the upwind cell's boundary stencil
-template <int PPM, int D, int SST>
-__device__ __forceinline__ double predict_special(const double* s, bool left, bool traced,
-                                                  double sig, int pos, int dlo, int dhi, int bclo,
-                                                  int bchi) {
-    const double* c = s + (left ? -SST : 0);
-    double w9[9], sm, sp;
-#pragma unroll
-    for (int o = -4; o <= 4; ++o) w9[4 + o] = (o >= -1 - PPM && o <= 1 + PPM) ? c[o * SST] : 0.0;
-    ppm_edges<PPM, D>(w9, pos - (left ? 1 : 0), dlo, dhi, bclo, bchi, sm, sp);
-    const double x = trace_face(c[0], left ? sp : sm, left ? sm : sp, sig);
-    return traced ? x : c[0];
-}
 
 // MODE, the boundary conditions of the domain sides in the tile's reach: 0: each
 // side is free of overrides or extrapolates to first order (or evenly), which
@@ -847,9 +770,11 @@ bool fused_edge_scal_ok(const mx_adv_ctx* c, int is_conservative) {
 // a tile and its stencil span at most 25 rows (32-bit byte offsets in a plane)
 bool fused_edge_rows_ok(const EdgeLevel& L) {
     const long long lim = 0x7fffffffLL / (8 * 26);
+    const long long max = 0x7fffffffLL;  // past which the launch refuses them
     auto ok = [&](const mx_multifab* m) {
         for (int b = 0; b < m->nfab; ++b)
-            if (m->fab[b].jstride > lim) return false;
+            if (m->fab[b].jstride > lim && m->fab[b].jstride <= max && m->fab[b].kstride <= max)
+                return false;
         return true;
     };
     bool r = ok(L.state) && ok(L.force);
@@ -936,6 +861,10 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
             act[d][0] = act[d][0] || bc_general(bcs[bccomps[vc]].lo[d], is_vel);
             act[d][1] = act[d][1] || bc_general(bcs[bccomps[vc]].hi[d], is_vel);
         }
+    auto clear_xy = [&](const FBox& B, int x, int nx, int y, int ny) {
+        return tile_clear(x, nx, B.domlo[0], B.domhi[0], act[0][0], act[0][1]) &&
+               tile_clear(y, ny, B.domlo[1], B.domhi[1], act[1][0], act[1][1]);
+    };
     const double dt = c->p.dt, dt2 = 0.5 * dt, dt3 = dt / 3.0, dt4 = 0.25 * dt, dt6 = dt / 6.0;
     const bool cons = is_conservative != 0;
     for (const EdgeLevel& L : levs) {
@@ -964,17 +893,26 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
             const DA* strided[] = {&B.s,     &B.fo,    &B.um[0], &B.um[1],
                                    &B.um[2], &B.se[0], &B.se[1], &B.se[2]};
             for (int q = 0; q < 8; ++q) B.ks[q] = 8 * strided[q]->ks;
+            for (const DA* d : strided)
+                if (d->js > 0x7fffffffLL || d->ks > 0x7fffffffLL) return MX_ERR_UNSUPPORTED;
             boxes.push_back(B);
             hb.push_back(g);
-            cols.push_back({g.hi[2] - g.lo[2] + 1, (long long)((g.hi[0] - g.lo[0] + TX) / TX) *
-                                                       ((g.hi[1] - g.lo[1] + TY) / TY)});
+            ChunkCols col{g.hi[2] - g.lo[2] + 1, {0, 0}};
+            for (int y = g.lo[1]; y <= g.hi[1]; y += TY)
+                for (int x = g.lo[0]; x <= g.hi[0]; x += TX)
+                    ++col.tiles[clear_xy(B, x, std::min(TX, g.hi[0] - x + 1), y,
+                                         std::min(TY, g.hi[1] - y + 1))
+                                    ? 0
+                                    : 1];
+            cols.push_back(col);
         }
     }
     if (tz <= 0) {
         const int per_cu = c->p.ppm_type == 1
                                ? (cons ? fused_blocks<1, true, TX, TY>() : fused_blocks<1, false, TX, TY>())
                                : (cons ? fused_blocks<2, true, TX, TY>() : fused_blocks<2, false, TX, TY>());
-        tz = pick_chunks(cols, num_comp, per_cu);
+        const int blocks[2] = {per_cu, std::min(per_cu, 3)};
+        tz = pick_chunks(cols, num_comp, blocks);
     }
     for (size_t id = 0; id < boxes.size(); ++id) {
         const HBox& g = hb[id];
@@ -992,11 +930,7 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
                             std::min(TY, g.hi[1] - y + 1),
                             ze - z,
                             0};
-                    const int t0[2] = {x, y}, tn[2] = {T.nx, T.ny};
-                    bool f = true;
-                    for (int d = 0; d < 2; ++d)
-                        f = f && tile_clear(t0[d], tn[d], B.domlo[d], B.domhi[d], act[d][0],
-                                            act[d][1]);
+                    const bool f = clear_xy(B, x, T.nx, y, T.ny);
                     for (int s = 0; s < 2; ++s)
                         if (!tile_clear(T.z0, T.nz, B.domlo[2], B.domhi[2], s == 0 && act[2][0],
                                         s == 1 && act[2][1]))

@@ -126,11 +126,12 @@ struct mx_adv_ctx {
     int utrans_chunks = 8; // chunks per y/z column of that form
     int vp_trans_all = 1;  // VelPred's transverse kernel: 1 = all six states per thread
     int vp_fused = 1;      // VelPred: 1 = the fused z-marching kernel where it applies
-    int vp_fused_tz = 32;  // planes per chunk of the fused VelPred kernel
+    int vp_fused_tz = 0;   // planes per chunk of the fused VelPred kernel; 0: pick_chunks
     int vp_fused_comp = 1; // fused VelPred: 1 = one velocity component per block
     int rhoh_flux_epilogue = 1;  // the pass: MakeRhoHFlux (planar, ept 0/1/3) in the
                                  // fused edge kernel's epilogue
-    int vp_fused_tile = 2; // its tile (waves per SIMD): 0 16x11 (3), 1 16x8 (3), 2 16x11 (4), 3 32x8 (3)
+    int vp_fused_tile = -1; // its tile (waves per SIMD): 0 16x11 (3), 1 16x8 (3), 2 16x11 (4), 3 32x8 (3),
+                            // 4 16x8 (4), 5 16x12 (4); -1: 2 for ppm_type 1, 0 for ppm_type 2
     int fused_tile = -1;    // 0: 32 x 8 columns, 1: 16 x 16, 2: 16 x 12, 3: 16 x 8,
                             // 4: 16 x 11; -1: 16 x 11
     int fused_per_box = 0;  // 1: one fused launch per box (comparison mode)
@@ -324,11 +325,12 @@ struct Table {
     }
 };
 
-// The z-marching kernels' chunks.  A level's tile columns by box: `tiles` columns
-// of `nz` planes; `nvar` blocks (components) per column chunk.
+// The z-marching kernels' chunks.  A level's tile columns by box: `nz` planes,
+// tiles[0] columns of a first launch and tiles[1] of a second one (those at
+// general sides); `nvar` blocks (components) per column chunk.
 struct ChunkCols {
     int nz;
-    long long tiles;
+    long long tiles[2];
 };
 // the number of chunks a box of nz planes is cut into for chunks of about tz, and
 // where chunk i of n starts: equal chunks, the longer ones first
@@ -337,7 +339,7 @@ inline int chunk_start(int nz, int n, int i) {
     const int q = nz / n, r = nz % n;
     return i * q + (i < r ? i : r);
 }
-int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, int blocks_per_cu);
+int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, const int blocks_per_cu[2]);
 
 // launch geometry: x covers the largest per-box region, y = boxes, z = extra
 inline dim3 grid_for(long long maxpts, int nbox, int nz, int block) {
