@@ -801,7 +801,7 @@ int mx_adv_scal_step(mx_adv_ctx* ctx, mx_fab* s, mx_fab* umac, mx_fab* snew, int
    dense (ncomp, n, n, n) arrays starting at index 0 are read in place.
    Piecewise differentiation: every limiter and upwind branch is taken as in
    the forward step.  Deterministic (no atomics); the workspace holds about
-   65 ncomp + 3 arrays of n^3 doubles. */
+   35 ncomp + 3 arrays of n^3 doubles. */
 int mx_adv_scal_step_vjp(mx_adv_ctx* ctx, mx_fab* s, mx_fab* umac, const mx_fab* gbar,
                          mx_fab* sbar, mx_fab* ubar, int ncomp, int is_conservative);
 
@@ -826,7 +826,7 @@ int mx_adv_scal_step_boxes(mx_adv_ctx* ctx, mx_multifab* s, mx_face_multifab* um
    lo..hi of umac (and the face at an outflow high side); no ghosts needed.
    The state adjoint of a cell on an outflow side includes the ghost cells
    that copy it.  Piecewise differentiation as in mx_adv_scal_step_vjp.
-   Deterministic.  Workspace: about 50 ncomp + 8 (ppm_type 2: 62 ncomp + 8)
+   Deterministic.  Workspace: about 35 ncomp + 8 (ppm_type 2: 47 ncomp + 8)
    arrays of the domain grown by 7 points per outflow direction. */
 int mx_adv_scal_step_vjp_boxes(mx_adv_ctx* ctx, const mx_multifab* s,
                                const mx_face_multifab* umac, const mx_multifab* gbar,

@@ -17,8 +17,8 @@
 // The adjoint differentiates the same arithmetic with every limiter and
 // upwind branch frozen at its forward value (the function is piecewise
 // smooth; at a switch point the derivative of the branch taken is used).
-// It runs as a tape of the forward intermediates (traced states, upwind
-// states, corner-coupled states, edge states, on dense periodic N^3 arrays)
+// It runs as a tape of the forward intermediates (upwind predictor states,
+// corner-coupled states, edge states, on dense periodic N^3 arrays)
 // and reverse sweeps that mirror the forward stages.  Every reverse stage
 // gathers the adjoints of its inputs from the adjoints of the outputs that
 // use them, so no atomics are used and the result is deterministic.
@@ -36,6 +36,7 @@
 #include <cstring>
 
 #include "mx_internal.H"
+#include "mx_march.H"
 
 using namespace mxd;
 using namespace mxh;
@@ -133,8 +134,8 @@ struct AB {
     const double* S;   // state, ncomp x N^3
     const double* U[3];
     const double* G;   // adjoint of snew
-    double *IP[3], *IM[3], *SIMH[3], *COR[6], *SE[3];
-    double *EB[6], *TB[3];
+    double *SIMH[3], *COR[6], *SE[3];
+    double *EB[3], *TB[3];  // EB[d]: of both edge terms that enter the d-face states
     double *SLB[3], *SRB[3];  // face sums (k_adj_fsum), when used
     double* UBC[3];           // per-component face velocity adjoints (k_adj_trace)
     double *S0S, *FLB[3], *FRB[3], *UHI[3], *ULO[3];  // S0S: trace terms of s, summed over d
@@ -149,7 +150,8 @@ struct AB {
     int xcd;           // the grid's x is a multiple of 8 and each XCD walks one
                        // contiguous eighth of it
     int fold;          // ghost reach of the state adjoint (general layout)
-    double dt, rel_eps, dx[3];
+    double dt, rel_eps;
+    DivBy dx[3];
     // per-direction factors, evaluated once on the host by the same
     // expressions: dt/h, (dt/4)/h (edge terms), (dt/6)/h (transverse terms);
     // the conservative form's (dt/2)/h (edge terms) and (dt/3)/h (transverse
@@ -187,7 +189,6 @@ __device__ __forceinline__ bool point(const AB& A, const PT& P, int& i, int& j, 
 // the foextrap rule at an outflow side (1: low, 2: high) for the predictor,
 // corner-coupled and edge states (MaestroMakeEdgeScalars.cpp:709-738,
 // :931-961, :1446-1480): the outside state takes the inside one
-__device__ __forceinline__ double upwind_b(double l, double r, double u, double thr, int b);
 // (selects, not branches: assignments under branches to the two
 // references put them in scratch memory)
 __device__ __forceinline__ void bfix(int b, double& wl, double& wr) {
@@ -211,47 +212,54 @@ __device__ __forceinline__ void weights(double u, double thr, double& wl, double
     }
 }
 
-__device__ __forceinline__ double upwind(double l, double r, double u, double thr) {
-    double res = (u > 0.0) ? l : r;
-    res = (dabs(u) > thr) ? res : 0.5 * (l + r);
-    return res;
-}
-
-__device__ __forceinline__ double upwind_b(double l, double r, double u, double thr, int b) {
-    const double L = b == 1 ? r : l;
-    const double R = b == 2 ? l : r;
-    return upwind(L, R, u, thr);
-}
+// a face's upwind choice (b: its outflow side, whose inside cell it takes):
+// `left` its low cell, else its high one, `both` their average.  One choice
+// serves every stage: a predictor state whose face velocity is within rel_eps
+// is its cell's plain value (ppm_trace), so the average is then of states that
+// start from the plain values, and every other state starts from the upwind
+// predictor state of its own face.
+struct Up {
+    bool left, both;
+    __device__ __forceinline__ Up(double u, double eps, int b) {
+        left = (u > 0.0 || b == 2) && b != 1;
+        both = !(dabs(u) > eps) && b == 0;
+    }
+};
 
 __device__ __forceinline__ double dabs_d(double x) { return signbit(x) ? -1.0 : 1.0; }
 
 // ---------------------------------------------------------------- forward tape
-// A1 + A2: traced PPM states of every cell and direction, and the upwind
-// state simh on the face below the cell (from the traced state of the cell
-// below it, recomputed here)
+// A1 + A2: the upwind predictor state simh on the low d-face of the cell: the
+// traced PPM state of the face's upwind cell only
 template <int PPM, int D, class PT>
-__device__ __forceinline__ void ppm_cell(const AB& A, const PT& P, const double* S, int i, int j,
-                                         int k, int pos, double& Ip, double& Im) {
+__device__ __forceinline__ double tape_dir(const AB& A, const PT& P, const double* S, int i, int j,
+                                           int k, long long p) {
+    const int pos = posd(D, i, j, k);
+    const double u = A.U[D][p];
+    const Up f(u, 0.0, P.bnd(D, pos));
+    const int sh = f.left ? 1 : 0;
     constexpr int G = PPM == 2 ? 3 : 2;
     double v[9];
 #pragma unroll
-    for (int o = -4; o <= 4; ++o) v[4 + o] = (o >= -G && o <= G) ? S[P.nb(i, j, k, D, o)] : 0.0;
+    for (int o = -4; o <= 4; ++o) v[4 + o] = (o >= -G && o <= G) ? S[P.nb(i, j, k, D, o - sh)] : 0.0;
     double sm, sp;
-    ppm_edges<PPM, D>(v, pos, 0, A.n - 1, MX_BC_INT_DIR, MX_BC_INT_DIR, sm, sp);
-    ppm_trace(v[4], sm, sp, A.U[D][P.nb(i, j, k, D, 1)], A.U[D][P.at(i, j, k)], A.dt, A.dx[D],
-              A.rel_eps, Ip, Im);
+    ppm_edges<PPM, D>(v, pos - sh, 0, A.n - 1, MX_BC_INT_DIR, MX_BC_INT_DIR, sm, sp);
+    const bool traced = f.left ? u > A.rel_eps : u < -A.rel_eps;
+    const double x = trace_face(v[4], f.left ? sp : sm, f.left ? sm : sp,
+                                div_by(dabs(u) * A.dt, A.dx[D]));
+    double h = traced ? x : v[4];
+    // at u = 0 the average of two untraced states (v[4] is the face's cell)
+    h = f.both ? 0.5 * (v[3] + v[4]) : h;
+    return h;
 }
 
-template <int PPM, int D, class PT>
-__device__ __forceinline__ void tape_dir(const AB& A, const PT& P, const double* S, int i, int j,
-                                         int k, long long p, double& ip, double& im, double& h) {
-    const int pos = D == 0 ? i : (D == 1 ? j : k);
-    ppm_cell<PPM, D>(A, P, S, i, j, k, pos, ip, im);
-    double ipm, imm;
-    ppm_cell<PPM, D>(A, P, S, i - (D == 0), j - (D == 1), k - (D == 2), pos - 1, ipm, imm);
-    h = upwind_b(ipm, im, A.U[D][p], 0.0, P.bnd(D, pos));
-}
-
+//
+// The tape's kernels are bound by the L1 path (its address and data units are
+// busy all the time, some 16 cycles per load and as many again on misses) and by
+// the limiters' FP64 work, so each evaluates a face's upwind cell only and keeps
+// one predictor state per face instead of both sides' and their choice.  128^3 of
+// 4 components, ppm_type 1, against both sides at every face: this kernel 265 ->
+// 150 us, the corner states 350 -> 250 us, the edge states 440 -> 340 us.
 template <int PPM, class PT>
 __global__ void __launch_bounds__(NTB) k_tape_ppm(AB A) {
     const PT P = PT::make(A);
@@ -260,18 +268,14 @@ __global__ void __launch_bounds__(NTB) k_tape_ppm(AB A) {
     if (!point(A, P, i, j, k, p)) return;
     const long long co = (long long)blockIdx.y * A.cs;
     const double* S = A.S + co;
-    double ip[3], imv[3], h[3];
-    tape_dir<PPM, 0>(A, P, S, i, j, k, p, ip[0], imv[0], h[0]);
-    tape_dir<PPM, 1>(A, P, S, i, j, k, p, ip[1], imv[1], h[1]);
-    tape_dir<PPM, 2>(A, P, S, i, j, k, p, ip[2], imv[2], h[2]);
+    double h[3];
+    h[0] = tape_dir<PPM, 0>(A, P, S, i, j, k, p);
+    h[1] = tape_dir<PPM, 1>(A, P, S, i, j, k, p);
+    h[2] = tape_dir<PPM, 2>(A, P, S, i, j, k, p);
     // every result is stored after the last load (stores and loads share
     // one in-order counter, so a load issued after a store waits for it)
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        A.IP[d][co + p] = ip[d];
-        A.IM[d][co + p] = imv[d];
-        A.SIMH[d][co + p] = h[d];
-    }
+    for (int d = 0; d < 3; ++d) A.SIMH[d][co + p] = h[d];
 }
 
 // MakeDivU of cell (i,j,k): the six face differences over dx[0]
@@ -309,15 +313,26 @@ __global__ void __launch_bounds__(NTB) k_tape_corner(AB A) {
     if (!point(A, P, i, j, k, p)) return;
     const long long co = (long long)blockIdx.y * A.cs;
     double cor[6];
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const int im = i - (d == 0), jm = j - (d == 1), km = k - (d == 2);
+        const int di = d == 0, dj = d == 1, dk = d == 2;
+        const Up f(A.U[d][p], A.rel_eps, P.bnd(d, posd(d, i, j, k)));
+        const double h = A.SIMH[d][co + p];
+        const int sh = f.left ? 1 : 0;
+#pragma unroll
         for (int t = 0; t < 3; ++t) {
             if (t == d) continue;
-            double l = A.IP[d][co + P.at(im, jm, km)];
-            double r = A.IM[d][co + p];
-            l = tcorr<CONS>(A, P, co, l, im, jm, km, t);
-            r = tcorr<CONS>(A, P, co, r, i, j, k, t);
-            cor[pidx(d, t)] = upwind_b(l, r, A.U[d][p], A.rel_eps, P.bnd(d, posd(d, i, j, k)));
+            cor[pidx(d, t)] = tcorr<CONS>(A, P, co, h, i - sh * di, j - sh * dj, k - sh * dk, t);
+        }
+        if (__builtin_expect(f.both, 0)) {
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                if (t == d) continue;
+                const double l = tcorr<CONS>(A, P, co, A.S[co + P.nb(i, j, k, d, -1)], i - di,
+                                             j - dj, k - dk, t);
+                const double r = tcorr<CONS>(A, P, co, A.S[co + p], i, j, k, t);
+                cor[pidx(d, t)] = 0.5 * (l + r);
+            }
         }
     }
     for (int q = 0; q < 6; ++q) A.COR[q][co + p] = cor[q];
@@ -368,23 +383,26 @@ __global__ void __launch_bounds__(NTB) k_tape_edge(AB A) {
     const long long co = (long long)blockIdx.y * A.cs;
     const double dt2 = 0.5 * A.dt;
     double se[3];
-    for (int d = 0; d < 3; ++d) {
-        const int im = i - (d == 0), jm = j - (d == 1), km = k - (d == 2);
-        double l = A.IP[d][co + P.at(im, jm, km)];
-        double r = A.IM[d][co + p];
+    // the state of cell (ci,cj,ck) on its d-face, from the predictor state x
+    auto state = [&](int d, double x, int ci, int cj, int ck) {
+#pragma unroll
         for (int t = 0; t < 3; ++t) {
             if (t == d) continue;
-            const int o = 3 - d - t;
-            l = l - et<CONS>(A, P, co, im, jm, km, t, o);
-            r = r - et<CONS>(A, P, co, i, j, k, t, o);
+            x = x - et<CONS>(A, P, co, ci, cj, ck, t, 3 - d - t);
         }
-        if (CONS) {
-            l = l - nterm(A, P, co, im, jm, km, d);
-            r = r - nterm(A, P, co, i, j, k, d);
+        if (CONS) x = x - nterm(A, P, co, ci, cj, ck, d);
+        return x + dt2 * 0.0;
+    };
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int di = d == 0, dj = d == 1, dk = d == 2;
+        const Up f(A.U[d][p], A.rel_eps, P.bnd(d, posd(d, i, j, k)));
+        const int sh = f.left ? 1 : 0;
+        se[d] = state(d, A.SIMH[d][co + p], i - sh * di, j - sh * dj, k - sh * dk);
+        if (__builtin_expect(f.both, 0)) {
+            const double l = state(d, A.S[co + P.nb(i, j, k, d, -1)], i - di, j - dj, k - dk);
+            se[d] = 0.5 * (l + state(d, A.S[co + p], i, j, k));
         }
-        const double sedgel = l + dt2 * 0.0;
-        const double sedger = r + dt2 * 0.0;
-        se[d] = upwind_b(sedgel, sedger, A.U[d][p], A.rel_eps, P.bnd(d, posd(d, i, j, k)));
     }
     // B1 (it needs only the output adjoint and the velocity): the flux,
     // update and edge-state upwinding give the per-cell edge-term adjoints;
@@ -400,15 +418,11 @@ __global__ void __launch_bounds__(NTB) k_tape_edge(AB A) {
         const double seb1 = edge_bar(A, P, co, i + (d == 0), j + (d == 1), k + (d == 2), d, wl1, wr1);
         lb1[d] = wl1 * seb1;
     }
-    for (int d = 0; d < 3; ++d) A.SE[d][co + p] = se[d];
 #pragma unroll
-    for (int t = 0; t < 3; ++t)
-#pragma unroll
-        for (int o = 0; o < 3; ++o) {
-            if (o == t) continue;
-            const int d = 3 - t - o;
-            A.EB[pidx(t, o)][co + p] = -lb1[d] - rb0[d];
-        }
+    for (int d = 0; d < 3; ++d) {
+        A.SE[d][co + p] = se[d];
+        A.EB[d][co + p] = -lb1[d] - rb0[d];
+    }
 }
 
 // ---------------------------------------------------------------- reverse
@@ -446,8 +460,8 @@ __device__ __forceinline__ void face_totals(const AB& A, const PT& P, long long 
     for (int o = 0; o < 3; ++o) {
         if (o == t) continue;
         const int q = pidx(t, o);
-        const double ebm = A.EB[q][co + fm];
-        const double eb0 = A.EB[q][co + f];
+        const double ebm = A.EB[3 - t - o][co + fm];
+        const double eb0 = A.EB[3 - t - o][co + f];
         const double kb = CONS ? ebm * b * u0 - eb0 * b * u0
                                : ebm * b * (u0 + um) - eb0 * b * (up + u0);
         if (want_u) {
@@ -481,8 +495,7 @@ __device__ __forceinline__ void face_totals(const AB& A, const PT& P, long long 
             const double sm = A.S[co + fm], s0 = A.S[co + f];
             const double tsm = A.TB[0][co + fm] + A.TB[1][co + fm] + A.TB[2][co + fm];
             const double ts0 = A.TB[0][co + f] + A.TB[1][co + f] + A.TB[2][co + f];
-            const int qn = t == 0 ? pidx(1, 2) : (t == 1 ? pidx(0, 2) : pidx(0, 1));
-            const double enm = A.EB[qn][co + fm], en0 = A.EB[qn][co + f];
+            const double enm = A.EB[t][co + fm], en0 = A.EB[t][co + f];
             ub = ub + (tbm * a * H[f] - tb0 * a * H[f]);
             ub = ub + (tb0 * a * s0 - tbm * a * sm);
             ub = ub + (A.dt3 / A.dx0) * (sm * tsm - s0 * ts0);
@@ -496,18 +509,19 @@ __device__ __forceinline__ void face_totals(const AB& A, const PT& P, long long 
     srb = srb + wr0 * hb;
 }
 
-// adjoint of the corner state q on d-face (i,j,k) (through the edge terms of
-// the cells on both sides of it), with its upwinding weights: the left and
+// adjoint of the corner state on d-face (i,j,k) corrected by o (through the
+// edge terms of the cells on both sides of it, which enter the states of the
+// third direction e = 3-d-o), with its upwinding weights: the left and
 // right predictor-state adjoints it passes on
 template <bool CONS, class PT>
 __device__ __forceinline__ void corner_bar(const AB& A, const PT& P, long long co, int i, int j,
-                                           int k, int d, int q, double& lb, double& rb) {
+                                           int k, int d, int e, double& lb, double& rb) {
     const double b = CONS ? A.f2[d] : A.f4[d];
     const long long c = P.at(i, j, k);
     const long long fm = P.nb(i, j, k, d, -1), fp = P.nb(i, j, k, d, 1);
     const double u0 = A.U[d][c], um = A.U[d][fm], up = A.U[d][fp];
-    const double ebm = A.EB[q][co + fm];
-    const double eb0 = A.EB[q][co + c];
+    const double ebm = A.EB[e][co + fm];
+    const double eb0 = A.EB[e][co + c];
     const double kb = CONS ? ebm * b * u0 - eb0 * b * u0
                            : ebm * b * (u0 + um) - eb0 * b * (up + u0);
     double wl, wr;
@@ -529,8 +543,7 @@ __device__ __forceinline__ double cons_direct(const AB& A, const PT& P, long lon
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
         const double du = A.U[t][P.nb(i, j, k, t, 1)] - A.U[t][c];
-        const int qn = t == 0 ? pidx(1, 2) : (t == 1 ? pidx(0, 2) : pidx(0, 1));
-        r += A.TB[t][co + c] * (A.dt3 * dv - A.f3[t] * du) + A.EB[qn][co + c] * (A.f2[t] * du);
+        r += A.TB[t][co + c] * (A.dt3 * dv - A.f3[t] * du) + A.EB[t][co + c] * (A.f2[t] * du);
     }
     return r;
 }
@@ -550,10 +563,10 @@ __global__ void __launch_bounds__(NTB) k_adj_tterm(AB A) {
         double s = 0.0;
         for (int d = 0; d < 3; ++d) {
             if (d == o) continue;
-            const int q = pidx(d, o);
+            const int e = 3 - d - o;
             double lb1, rb1, lb0, rb0;
-            corner_bar<CONS>(A, P, co, i + (d == 0), j + (d == 1), k + (d == 2), d, q, lb1, rb1);
-            corner_bar<CONS>(A, P, co, i, j, k, d, q, lb0, rb0);
+            corner_bar<CONS>(A, P, co, i + (d == 0), j + (d == 1), k + (d == 2), d, e, lb1, rb1);
+            corner_bar<CONS>(A, P, co, i, j, k, d, e, lb0, rb0);
             s += lb1 + rb0;
         }
         tb[o] = -s;
@@ -587,30 +600,30 @@ struct TraceBar {
     double smb, spb, s0b, uhib, ulob;
 };
 __device__ __forceinline__ TraceBar trace_bar(const AB& A, double s0, double sm, double sp,
-                                              double s6, double uhi, double ulo, double h,
+                                              double s6, double uhi, double ulo, const DivBy& h,
                                               double Ipb, double Imb) {
     TraceBar r = {0.0, 0.0, 0.0, 0.0, 0.0};
     if (uhi > A.rel_eps) {
-        const double sg = dabs(uhi) * A.dt / h;
+        const double sg = div_by(dabs(uhi) * A.dt, h);
         const double f = 1.0 - C23 * sg;
         const double Aq = sp - sm - f * s6;
         r.spb += Ipb * (1.0 - 0.5 * sg * (1.0 + 3.0 * f));
         r.smb += Ipb * (-0.5 * sg * (-1.0 + 3.0 * f));
         r.s0b += Ipb * (3.0 * sg * f);
         const double sgb = Ipb * (-0.5 * Aq - 0.5 * sg * (C23 * s6));
-        r.uhib += sgb * dabs_d(uhi) * A.dt / h;
+        r.uhib += div_by(sgb * dabs_d(uhi) * A.dt, h);
     } else {
         r.s0b += Ipb;
     }
     if (ulo < -A.rel_eps) {
-        const double sg = dabs(ulo) * A.dt / h;
+        const double sg = div_by(dabs(ulo) * A.dt, h);
         const double f = 1.0 - C23 * sg;
         const double Bq = sp - sm + f * s6;
         r.smb += Imb * (1.0 + 0.5 * sg * (-1.0 - 3.0 * f));
         r.spb += Imb * (0.5 * sg * (1.0 - 3.0 * f));
         r.s0b += Imb * (3.0 * sg * f);
         const double sgb = Imb * (0.5 * Bq - 0.5 * sg * (C23 * s6));
-        r.ulob += sgb * dabs_d(ulo) * A.dt / h;
+        r.ulob += div_by(sgb * dabs_d(ulo) * A.dt, h);
     } else {
         r.s0b += Imb;
     }
@@ -639,10 +652,10 @@ __global__ void __launch_bounds__(NTB) k_adj_trace(AB A) {
         const double dl = vl_slope(v[2], v[3], v[4]);
         const double dc = vl_slope(v[3], v[4], v[5]);
         const double dr = vl_slope(v[4], v[5], v[6]);
-        double sm0 = 0.5 * (v[4] + v[3]) - (dc - dl) / 6.0;
+        double sm0 = 0.5 * (v[4] + v[3]) - div6(dc - dl);
         sm0 = dmax(sm0, dmin(v[4], v[3]));
         sm0 = dmin(sm0, dmax(v[4], v[3]));
-        double sp0 = 0.5 * (v[5] + v[4]) - (dr - dc) / 6.0;
+        double sp0 = 0.5 * (v[5] + v[4]) - div6(dr - dc);
         sp0 = dmax(sp0, dmin(v[5], v[4]));
         sp0 = dmin(sp0, dmax(v[5], v[4]));
         const double s0 = v[4];
@@ -663,7 +676,7 @@ __global__ void __launch_bounds__(NTB) k_adj_trace(AB A) {
         }
         const long long fhi = P.nb(i, j, k, d, 1);
         const double uhi = A.U[d][fhi], ulo = A.U[d][p];
-        const double h = A.dx[d];
+        const DivBy& h = A.dx[d];
         const double s6 = 6.0 * s0 - 3.0 * (sm + sp);
         double Ipb, Imb;
         if (FS) {
@@ -766,10 +779,10 @@ __device__ __forceinline__ void cs_face_grad(double sa, double sb, double sc, do
                 l[0] = 0.5; l[1] = -0.5; l[2] = -0.5; l[3] = 0.5;          // D2
             }
         }
-        g[0] = -l[0] / 6.0;
-        g[1] = 0.5 - l[1] / 6.0;
-        g[2] = 0.5 - l[2] / 6.0;
-        g[3] = -l[3] / 6.0;
+        g[0] = -div6(l[0]);
+        g[1] = 0.5 - div6(l[1]);
+        g[2] = 0.5 - div6(l[2]);
+        g[3] = -div6(l[3]);
     }
 }
 
@@ -1041,7 +1054,7 @@ __device__ __forceinline__ void face_bar(const AB& A, const PT& P, long long co,
     const double sa = S[cm], sb = S[c];
     const double sa2 = S[P.nb(i, j, k, d, -2)], sb2 = S[P.nb(i, j, k, d, 1)];
     const double dla = vl_slope(sa2, sa, sb), dlb = vl_slope(sa, sb, sb2);
-    const double e0 = 0.5 * (sb + sa) - (dlb - dla) / 6.0;
+    const double e0 = 0.5 * (sb + sa) - div6(dlb - dla);
     const double m1 = dmin(sb, sa);
     const bool m1a = sa < sb;  // dmin(sb, sa) returns sa
     const double e1 = dmax(e0, m1);
@@ -1061,8 +1074,8 @@ __device__ __forceinline__ void face_bar(const AB& A, const PT& P, long long co,
     } else {
         bsa = 0.5 * eb;
         bsb = 0.5 * eb;
-        bla = eb / 6.0;
-        blb = -eb / 6.0;
+        bla = div6(eb);
+        blb = -bla;
     }
 }
 
@@ -1384,8 +1397,6 @@ long long ab_arrays(const mx_adv_ctx* c, AB& A, int ncomp, bool gen, Take take) 
         n += ncomp;
     };
     for (int d = 0; d < 3; ++d) {
-        t(A.IP[d]);
-        t(A.IM[d]);
         t(A.SIMH[d]);
         t(A.SE[d]);
         t(A.TB[d]);
@@ -1410,10 +1421,8 @@ long long ab_arrays(const mx_adv_ctx* c, AB& A, int ncomp, bool gen, Take take) 
             t(A.QP[d]);
         }
     }
-    for (int q = 0; q < 6; ++q) {
-        t(A.COR[q]);
-        t(A.EB[q]);
-    }
+    for (int d = 0; d < 3; ++d) t(A.EB[d]);
+    for (int q = 0; q < 6; ++q) t(A.COR[q]);
     t(A.S0S);
     return n;
 }
@@ -1426,12 +1435,13 @@ void ab_factors(const mx_adv_ctx* c, AB& A, int ncomp) {
     A.dt3 = dt3;
     A.dx0 = c->p.dx[0][0];
     for (int d = 0; d < 3; ++d) {
-        A.dx[d] = c->p.dx[0][d];
-        A.fdt[d] = A.dt / A.dx[d];
-        A.f4[d] = dt4 / A.dx[d];
-        A.f6[d] = dt6 / A.dx[d];
-        A.f2[d] = dt2 / A.dx[d];
-        A.f3[d] = dt3 / A.dx[d];
+        const double h = c->p.dx[0][d];
+        A.dx[d] = div_const(h);
+        A.fdt[d] = A.dt / h;
+        A.f4[d] = dt4 / h;
+        A.f6[d] = dt6 / h;
+        A.f2[d] = dt2 / h;
+        A.f3[d] = dt3 / h;
     }
 }
 
