@@ -72,6 +72,7 @@ constexpr int fused_wpe(int ppm, bool cons, int tx, int ty, int mode) {
 
 struct FBox {
     int hi[3];
+    int pad_ = 0;  // explicit, so that equal tables are equal byte for byte
     DA s, fo;
     DA um[3], se[3];
     // plane strides in bytes: s, force, umac x / y / z, sedge x / y / z

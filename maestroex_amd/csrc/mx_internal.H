@@ -372,9 +372,16 @@ int fill_patch_uedge(mx_adv_ctx* c, int nlev, const mx_face_multifab* uedge);
 // the workspace VelPred's temporaries need on one level
 size_t velpred_ws_bytes(const mx_adv_ctx* c, int lev);
 int check_phys(const mx_adv_ctx* c);
+// Addw0 (mult = 1) as part of the store of MakeUtrans' and VelPred's faces.
+// planar: the level's w0, added to the vertical faces; spherical: w0mac, which
+// the boxes hold already
+struct W0Add {
+    bool utrans = false, umac = false;
+    const double* w0 = nullptr;
+};
 int make_utrans(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_multifab* ufull,
                 const mx_face_multifab* utrans, const mx_face_multifab* w0mac,
-                const mx_multifab* w0_cart, bool fill = true);
+                const mx_multifab* w0_cart, bool fill = true, const W0Add& add = {});
 // fused 3-D VelPred (ppm_type 1/2, forces not traced): the boxes of every
 // listed level in one launch
 struct VpLevel {
@@ -386,9 +393,12 @@ struct VpLevel {
     const mx_face_multifab* w0mac;
     const mx_multifab* force;
     const mx_multifab* w0_cart;
+    W0Add add = {};
 };
 bool velpred_fused_ok(const mx_adv_ctx* c);
-int velpred_fused(mx_adv_ctx* c, const std::vector<VpLevel>& levs);
+// added: set where the kernel has added w0 as the levels' `add` asks (the
+// all-components kernel does not)
+int velpred_fused(mx_adv_ctx* c, const std::vector<VpLevel>& levs, bool* added = nullptr);
 int velpred(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_multifab* ufull,
             const mx_face_multifab* utrans, const mx_face_multifab* umac,
             const mx_face_multifab* w0mac, const mx_multifab* force, const mx_multifab* w0_cart);
@@ -406,7 +416,8 @@ struct VpPlan {
 int velpred_setup(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_multifab* ufull,
                   const mx_face_multifab* utrans, const mx_face_multifab* umac,
                   const mx_face_multifab* w0mac, const mx_multifab* force,
-                  const mx_multifab* w0_cart, VpPlan& plan, bool reserve = true);
+                  const mx_multifab* w0_cart, VpPlan& plan, bool reserve = true,
+                  const W0Add& add = {});
 int utrans_from_plan(mx_adv_ctx* c, const VpPlan& plan, bool fill = true);
 int velpred_finish(mx_adv_ctx* c, const VpPlan& plan);
 int make_edge_scal(mx_adv_ctx* c, int lev, const mx_multifab* state,

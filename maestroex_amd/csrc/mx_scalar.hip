@@ -946,6 +946,33 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
     // between levels; a single level fills its ghost faces on its own
     const bool multi = nlev > 1;
     if (multi && lev0 != 0) return MX_ERR_ARG;
+    // Addw0 where utrans and umac are stored, where that leaves every ghost
+    // face what Addw0's own pass makes it.  Spherical: that pass touches valid
+    // faces only, and umac has no ghost fill before it.  Planar: it also adds to
+    // the vertical faces' transverse ghosts, all of which the fill that follows
+    // rewrites if those directions are periodic and the level (or, below a finer
+    // one, level 0) leaves no gap; the ghost fill between MakeUtrans and Addw0
+    // then does nothing that the one after Addw0 does not repeat.  (With walls
+    // in two directions it does: FillUmacGhost's x and y steps each read corners
+    // that the other writes.)
+    bool w0_fold = true;
+    if (!sph) {
+        for (int d = 0; d < p.dim - 1; ++d)
+            w0_fold = w0_fold && p.is_periodic[d] && p.phys_bc_lo[d] == MX_PHYS_INTERIOR &&
+                      p.phys_bc_hi[d] == MX_PHYS_INTERIOR;
+        if (multi) {
+            long long cells = 0, dom = 1;
+            for (const mx_box& b : c->grids[0]) cells += npts(hbox(b));
+            for (int d = 0; d < p.dim; ++d) dom *= p.domain_hi[0][d] - p.domain_lo[0][d] + 1;
+            w0_fold = w0_fold && cells == dom;
+        }
+    }
+    std::vector<W0Add> w0a(nlev);
+    for (int i = 0; i < nlev; ++i) {
+        w0a[i].utrans = w0_fold && (multi || !sph);
+        w0a[i].umac = w0_fold;
+        if (!sph) w0a[i].w0 = a[i].w0.p + (long long)(lev0 + i) * a[i].w0.len;
+    }
     std::vector<VpPlan> vps(nlev);
     // the fused VelPred kernel keeps its temporaries on chip: MakeUtrans
     // reconstructs its own normal states and VelPred follows in one launch
@@ -954,7 +981,7 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
     for (int i = 0; i < nlev && vfused; ++i) {
         const mx_adv_pass_args* A = &a[i];
         vlevs.push_back({lev0 + i, &A->utilde, &A->ufull, &A->utrans, &A->umac, &A->w0mac,
-                         &A->vel_force, &A->w0_cart});
+                         &A->vel_force, &A->w0_cart, w0a[i]});
     }
     if (multi && !vfused) {
         // every level's VelPred temporaries stay live until the levels'
@@ -963,32 +990,41 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
         for (int i = 0; i < nlev; ++i) need += velpred_ws_bytes(c, lev0 + i);
         if ((rc = ws_reserve(c, need))) return rc;
     }
+    // Addw0's own pass (added: it was part of the store), and on a single level
+    // the ghost faces
+    auto add_w0 = [&](int i, const mx_face_multifab* f, bool added) -> int {
+        if (!added) return addw0(c, lev0 + i, f, &a[i].w0mac, &a[i].w0, 1.0, !multi);
+        return multi ? MX_OK : fill_face_ghosts(c, lev0 + i, f);
+    };
     for (int i = 0; i < nlev && vfused; ++i) {
         const int lev = lev0 + i;
         const mx_adv_pass_args* A = &a[i];
+        const bool add = w0a[i].utrans;
         if ((rc = make_utrans(c, lev, &A->utilde, &A->ufull, &A->utrans, &A->w0mac, &A->w0_cart,
-                              !multi)))
+                              !multi && !add, w0a[i])))
             return rc;
-        if ((rc = addw0(c, lev, &A->utrans, &A->w0mac, &A->w0, 1.0, !multi))) return rc;
+        if ((rc = add_w0(i, &A->utrans, add))) return rc;
         if (multi) continue;
         std::vector<VpLevel> one(1, vlevs[i]);
-        if ((rc = velpred_fused(c, one))) return rc;
-        if ((rc = addw0(c, lev, &A->umac, &A->w0mac, &A->w0, 1.0))) return rc;
+        bool added;
+        if ((rc = velpred_fused(c, one, &added))) return rc;
+        if ((rc = add_w0(i, &A->umac, added && w0a[i].umac))) return rc;
     }
     for (int i = 0; i < nlev && !vfused; ++i) {
         const int lev = lev0 + i;
         const mx_adv_pass_args* A = &a[i];
+        const bool add = w0a[i].utrans;
         // VelPred's reconstruction runs first and MakeUtrans reads its traced
         // normal-direction states (the numbers MakeUtrans would compute)
         VpPlan& vp = vps[i];
         if ((rc = velpred_setup(c, lev, &A->utilde, &A->ufull, &A->utrans, &A->umac, &A->w0mac,
-                                &A->vel_force, &A->w0_cart, vp, !multi)))
+                                &A->vel_force, &A->w0_cart, vp, !multi, w0a[i])))
             return rc;
-        if ((rc = utrans_from_plan(c, vp, !multi))) return rc;
-        if ((rc = addw0(c, lev, &A->utrans, &A->w0mac, &A->w0, 1.0, !multi))) return rc;
+        if ((rc = utrans_from_plan(c, vp, !multi && !add))) return rc;
+        if ((rc = add_w0(i, &A->utrans, add))) return rc;
         if (multi) continue;
         if ((rc = velpred_finish(c, vp))) return rc;
-        if ((rc = addw0(c, lev, &A->umac, &A->w0mac, &A->w0, 1.0))) return rc;
+        if ((rc = add_w0(i, &A->umac, w0a[i].umac))) return rc;
     }
     // AverageDownFaces over the hierarchy, then FillPatchUedge
     auto sync_levels = [&](mx_face_multifab mx_adv_pass_args::*field, bool fill) -> int {
@@ -1008,11 +1044,12 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
         // the first one wrote, so one sync after the w0 addition gives the
         // same values.
         if ((rc = sync_levels(&mx_adv_pass_args::utrans, true))) return rc;
-        if (vfused && (rc = velpred_fused(c, vlevs))) return rc;
+        bool added = true;
+        if (vfused && (rc = velpred_fused(c, vlevs, &added))) return rc;
         for (int i = 0; i < nlev; ++i) {
             const mx_adv_pass_args* A = &a[i];
             if (!vfused && (rc = velpred_finish(c, vps[i]))) return rc;
-            if ((rc = addw0(c, lev0 + i, &A->umac, &A->w0mac, &A->w0, 1.0, false))) return rc;
+            if ((rc = add_w0(i, &A->umac, added && w0a[i].umac))) return rc;
         }
         if ((rc = sync_levels(&mx_adv_pass_args::umac, true))) return rc;
     }

@@ -36,15 +36,34 @@ struct UtBox {
     DA ut, uf, w0c;
     DA tr[3];
     DA w0m[3];
+    const double* w0a;  // Addw0 at the store: the planar w0
+    int add;            // and which faces take it: bit 0 utrans, bit 1 umac
+    int pad_ = 0;       // explicit, so that equal tables are equal byte for byte
 };
 
 struct UtArgs {
     int bclo[3][3], bchi[3][3];  // bcs_u[comp].lo/hi[dir]
 };
 
+// Addw0 of a D-face where it is stored (a pass of its own reads and writes the
+// face again: 139 of 5450 us for utrans and umac of 256^3)
+enum { ADD_UTRANS = 1, ADD_UMAC = 2 };
 template <int D, class BOX>
-__device__ __forceinline__ void utrans_riemann(const BOX& B, const KGeom& g, int i, int j, int k,
-                                               double ul, double ur);
+__device__ __forceinline__ double plus_w0(const BOX& B, const KGeom& g, int which, int i, int j,
+                                          int k, double x) {
+    if (!(B.add & which)) return x;
+    if (g.spherical) return x + B.w0m[D](i, j, k);
+    return D == g.dim - 1 ? x + B.w0a[g.dim == 2 ? j : k] : x;
+}
+template <class BOX>
+void set_w0(BOX& B, const W0Add& add) {
+    B.w0a = add.w0;
+    B.add = (add.utrans ? ADD_UTRANS : 0) | (add.umac ? ADD_UMAC : 0);
+}
+
+template <int D, class BOX>
+__device__ __forceinline__ double utrans_riemann(const BOX& B, const KGeom& g, int i, int j, int k,
+                                                 double ul, double ur);
 
 template <int PPM, int D>
 __device__ __forceinline__ void utrans_face(const UtBox& B, const KGeom& g, const UtArgs& A,
@@ -79,15 +98,16 @@ __device__ __forceinline__ void utrans_face(const UtBox& B, const KGeom& g, cons
         ur = Im;
     }
 
-    utrans_riemann<D>(B, g, i, j, k, ul, ur);
+    const double x = utrans_riemann<D>(B, g, i, j, k, ul, ur);
+    B.tr[D](i, j, k) = plus_w0<D>(B, g, ADD_UTRANS, i, j, k, x);
 }
 
 // the PhysBC overrides and the Riemann solve of MakeUtrans on D-face
 // (i, j, k) from its left and right states (MaestroMakeUtrans.cpp:109-150,
 // 253-266); BOX: any box descriptor with ut, w0c, w0m and tr views
 template <int D, class BOX>
-__device__ __forceinline__ void utrans_riemann(const BOX& B, const KGeom& g, int i, int j, int k,
-                                               double ul, double ur) {
+__device__ __forceinline__ double utrans_riemann(const BOX& B, const KGeom& g, int i, int j, int k,
+                                                 double ul, double ur) {
     const int im = i - e(D, 0), jm = j - e(D, 1), km = k - e(D, 2);
     const int pos = D == 0 ? i : (D == 1 ? j : k);
     if (pos == g.domlo[D]) {
@@ -151,7 +171,7 @@ __device__ __forceinline__ void utrans_riemann(const BOX& B, const KGeom& g, int
         res = 0.5 * (ul + ur) > 0.0 ? ul : ur;
         res = test ? 0.0 : res;
     }
-    B.tr[D](i, j, k) = res;
+    return res;
 }
 
 template <int PPM>
@@ -193,7 +213,7 @@ __global__ void __launch_bounds__(256) k_utrans(const UtBox* __restrict__ boxes,
 //     takes ppm_edges in full where the cell has a boundary stencil.
 constexpr int UT_NT = 256;
 
-template <int PPM>
+template <int PPM, int ADD>
 __device__ __forceinline__ void utrans_rows(const UtBox& B, const KGeom& g, const UtArgs& A) {
     const unsigned nx = (unsigned)(B.hi[0] - B.lo[0] + 1);
     const unsigned ny = (unsigned)(B.hi[1] - B.lo[1] + 1);
@@ -220,10 +240,14 @@ __device__ __forceinline__ void utrans_rows(const UtBox& B, const KGeom& g, cons
     }
     // every lane takes part in the shuffle; lane 0's result is unused
     const double Ipl = __shfl_up(Ip, 1u, 64);
-    if (on && lane > 0 && c > 0) utrans_riemann<0>(B, g, i, j, k, Ipl, Im);
+    if (on && lane > 0 && c > 0) {
+        double x = utrans_riemann<0>(B, g, i, j, k, Ipl, Im);
+        if (ADD == 2) x = x + B.w0m[0](i, j, k);
+        B.tr[0](i, j, k) = x;
+    }
 }
 
-template <int PPM, int D>
+template <int PPM, int D, int ADD>
 __device__ __forceinline__ void utrans_march(const UtBox& B, const KGeom& g, const UtArgs& A,
                                              int nch) {
     constexpr int G = PPM == 2 ? 3 : 2;
@@ -250,6 +274,10 @@ __device__ __forceinline__ void utrans_march(const UtBox& B, const KGeom& g, con
     double Ipl = 0.0;
     double zf0 = 0.0, zf1 = 0.0, zf2 = 0.0, zsl = 0.0;
     for (int cpos = f0 - 1;; ++cpos) {
+        // Addw0's planar w0 of this face, before the loads that are not yet
+        // waited for
+        double wa = 0.0;
+        if (ADD == 1 && D == 2) wa = B.w0a[max(cpos, f0)];
         // the next cell's window entry and velocity, loaded ahead
         double vn = 0.0, un = 0.0;
         if (cpos < f1) {
@@ -285,7 +313,13 @@ __device__ __forceinline__ void utrans_march(const UtBox& B, const KGeom& g, con
             ppm_edges<PPM, D>(v, cpos, dlo, dhi, bclo, bchi, sm, sp);
         if (PPM == 1) zf0 = zf1;
         ppm_trace(v[4], sm, sp, uc, uc, g.dt, g.dx[D], g.rel_eps, Ip, Im);
-        if (cpos >= f0) utrans_riemann<D>(B, g, i, D == 1 ? cpos : tt, D == 2 ? cpos : tt, Ipl, Im);
+        if (cpos >= f0) {
+            const int j = D == 1 ? cpos : tt, k = D == 2 ? cpos : tt;
+            double x = utrans_riemann<D>(B, g, i, j, k, Ipl, Im);
+            if (ADD == 1 && D == 2) x = x + wa;
+            if (ADD == 2) x = x + B.w0m[D](i, j, k);
+            B.tr[D](i, j, k) = x;
+        }
         if (cpos == f1) break;
         Ipl = Ip;
 #pragma unroll
@@ -297,16 +331,20 @@ __device__ __forceinline__ void utrans_march(const UtBox& B, const KGeom& g, con
     }
 }
 
-template <int PPM>
-__global__ void __launch_bounds__(UT_NT) k_utrans_line(const UtBox* __restrict__ boxes, KGeom g,
-                                                      UtArgs A, int nch) {
+// ADD: Addw0 in the store, 0 no, 1 planar (z-faces), 2 spherical.  The register
+// budgets are what the kernel takes without it (two more lose a wave per SIMD:
+// 526 -> 590 us on 256^3, ppm_type 2)
+template <int PPM, int ADD>
+__global__ void __launch_bounds__(UT_NT)
+    __attribute__((amdgpu_waves_per_eu(PPM == 2 ? 5 : 6))) k_utrans_line(const UtBox* __restrict__ boxes, KGeom g, UtArgs A,
+                                                                          int nch) {
     const UtBox& B = boxes[blockIdx.y];
     if (blockIdx.z == 0)
-        utrans_rows<PPM>(B, g, A);
+        utrans_rows<PPM, ADD>(B, g, A);
     else if (blockIdx.z == 1)
-        utrans_march<PPM, 1>(B, g, A, nch);
+        utrans_march<PPM, 1, ADD>(B, g, A, nch);
     else
-        utrans_march<PPM, 2>(B, g, A, nch);
+        utrans_march<PPM, 2, ADD>(B, g, A, nch);
 }
 
 // ---------------------------------------------------------------------------
@@ -319,6 +357,9 @@ struct VpBox {
     DA Ip[3], Im[3];    // per velocity component: [dir] comps; ppm_type 0: slopes along dir
     DA Ipf[3], Imf[3];  // traced forces
     DA T[6];            // transverse states, pair_index(d, t)
+    const double* w0a;  // Addw0 at the store, as in UtBox
+    int add;
+    int pad_ = 0;
 };
 
 struct VpArgs {
@@ -735,7 +776,7 @@ __device__ __forceinline__ void vp_vel(const VpBox& B, const KGeom& g, int i, in
             default: break;
         }
     }
-    B.um[D](i, j, k) = res;
+    B.um[D](i, j, k) = plus_w0<D>(B, g, ADD_UMAC, i, j, k, res);
 }
 
 __global__ void __launch_bounds__(256) k_vp_vel(const VpBox* __restrict__ boxes, KGeom g) {
@@ -776,7 +817,8 @@ __device__ __forceinline__ void utrans_pp_face(const VpBox& B, const KGeom& g, i
         ul = B.Ip[D](im, jm, km, D);
         ur = B.Im[D](i, j, k, D);
     }
-    utrans_riemann<D>(B, g, i, j, k, ul, ur);
+    const double x = utrans_riemann<D>(B, g, i, j, k, ul, ur);
+    B.tr[D](i, j, k) = plus_w0<D>(B, g, ADD_UTRANS, i, j, k, x);
 }
 
 template <int PPM>
@@ -813,7 +855,7 @@ int check_phys(const mx_adv_ctx* c) {
 
 int make_utrans(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_multifab* ufull,
                 const mx_face_multifab* utrans, const mx_face_multifab* w0mac,
-                const mx_multifab* w0_cart, bool fill) {
+                const mx_multifab* w0_cart, bool fill, const W0Add& add) {
     const int dim = c->p.dim;
     const auto& grids = c->grids[lev];
     const bool sph = dim == 3 && c->p.spherical;
@@ -833,6 +875,7 @@ int make_utrans(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_mult
             B.tr[d] = d < dim ? to_da(utrans->dir[d].fab[b]) : null_da();
             B.w0m[d] = (sph && d < dim) ? to_da(w0mac->dir[d].fab[b]) : null_da();
         }
+        set_w0(B, add);
         // the grid covers the largest face region of any direction
         for (int d = 0; d < dim; ++d) maxpts = std::max(maxpts, npts(nodal(g, d)));
         boxes.push_back(B);
@@ -869,10 +912,18 @@ int make_utrans(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_mult
     const UtBox* dp = tab.dev<UtBox>(off);
     dim3 gr = grid_for(maxpts, (int)boxes.size(), dim, block);
     const dim3 gl((unsigned)lblocks, (unsigned)boxes.size(), 3);
-    if (line && c->p.ppm_type == 1)
-        MX_LAUNCH(c, "k_utrans", k_utrans_line<1>, gl, dim3(UT_NT), dp, kg, A, nch);
-    else if (line)
-        MX_LAUNCH(c, "k_utrans", k_utrans_line<2>, gl, dim3(UT_NT), dp, kg, A, nch);
+    auto line_launch = [&](auto w0_kind) {
+        constexpr int ADD = decltype(w0_kind)::value;
+        if (c->p.ppm_type == 1)
+            MX_LAUNCH(c, "k_utrans", (k_utrans_line<1, ADD>), gl, dim3(UT_NT), dp, kg, A, nch);
+        else
+            MX_LAUNCH(c, "k_utrans", (k_utrans_line<2, ADD>), gl, dim3(UT_NT), dp, kg, A, nch);
+        return MX_OK;
+    };
+    if (line)
+        rc = !add.utrans ? line_launch(std::integral_constant<int, 0>{})
+             : sph       ? line_launch(std::integral_constant<int, 2>{})
+                         : line_launch(std::integral_constant<int, 1>{});
     else if (c->p.ppm_type == 0)
         MX_LAUNCH(c, "k_utrans", k_utrans<0>,  gr, dim3(block), dp, kg, A);
     else if (c->p.ppm_type == 1)
@@ -880,13 +931,14 @@ int make_utrans(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_mult
     else
         MX_LAUNCH(c, "k_utrans", k_utrans<2>,  gr, dim3(block), dp, kg, A);
 
+    if (rc) return rc;
     return fill ? fill_face_ghosts(c, lev, utrans) : MX_OK;
 }
 
 int velpred_setup(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_multifab* ufull,
                   const mx_face_multifab* utrans, const mx_face_multifab* umac,
                   const mx_face_multifab* w0mac, const mx_multifab* force,
-                  const mx_multifab* w0_cart, VpPlan& plan, bool reserve) {
+                  const mx_multifab* w0_cart, VpPlan& plan, bool reserve, const W0Add& add) {
     const int dim = c->p.dim;
     const auto& grids = c->grids[lev];
     const bool sph = dim == 3 && c->p.spherical;
@@ -939,6 +991,7 @@ int velpred_setup(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_mu
             B.Imf[d] = (tf && d < dim) ? Imf[d][b] : null_da();
         }
         for (int p = 0; p < 6; ++p) B.T[p] = dim == 3 ? T[p][b] : null_da();
+        set_w0(B, add);
         maxpts = std::max(maxpts, npts(grown1(g)));
         boxes.push_back(B);
     }

@@ -66,6 +66,9 @@ struct VFBox {
     // z, w0mac x / y / z, w0_cart; the cell widths as divisors
     long long ks[13];
     DivBy h[3];
+    const double* w0a;  // Addw0 at the store of umac: the planar w0
+    int add;
+    int pad_ = 0;  // explicit, so that equal tables are equal byte for byte
 };
 
 struct VFTile {
@@ -867,6 +870,7 @@ struct VPLayout {
 };
 
 typedef __attribute__((address_space(4))) const VFBox cvbox;
+typedef __attribute__((address_space(4))) const double cd4;
 __device__ __forceinline__ cvbox* vfresh(const VFBox* p) {
     unsigned long long a = (unsigned long long)p;
     asm("" : "+s"(a));
@@ -977,6 +981,8 @@ __device__ __forceinline__ void vp_comp(const VFBox& B, const VPTile& tl, const 
     // (utrans_N stands in, so that the load is unconditional).  It has no ghosts
     // that the tile's own faces do not lie in.
     const bool has_w = sph || N == 2;
+    const bool add_m = sph && B.add, add_p = !sph && B.add;
+    cd4* const w0_z = (cd4*)B.w0a;
     const DA wv = sph ? B.w0m[N] : (N == 2 ? B.w0c : B.tr[N]);
     const int aw = min(max(a, 1), N == 0 ? nx + 1 : nx), bw = min(max(b, 1), N == 1 ? ny + 1 : ny);
     const unsigned oWv = (unsigned)(aw - 1) * 8u + (unsigned)(bw - 1) * (unsigned)wv.js * 8u;
@@ -1127,6 +1133,9 @@ __device__ __forceinline__ void vp_comp(const VFBox& B, const VPTile& tl, const 
             }
         }
         const bool now = N < 2 ? q >= z0 + 2 : q > z0 && (q <= z1 + 1 || last_z);
+        // Addw0: w0mac, or the planar w0 of z-face q - 1
+        if (add_m) res = res + w_r;
+        if (N == 2 && add_p) res = res + w0_z[now ? q - 1 : z0];
         if (now && store) gstore(oP, oO, res);
     };
     sN += B.ks[0];
@@ -1460,6 +1469,8 @@ int vf_boxes(mx_adv_ctx* c, const std::vector<VpLevel>& levs, std::vector<VFBox>
             }
             const DA* views[] = {&B.ut,    &B.fo,    &B.uf,     &B.tr[0],  &B.tr[1],  &B.tr[2], &B.um[0],
                                  &B.um[1], &B.um[2], &B.w0m[0], &B.w0m[1], &B.w0m[2], &B.w0c};
+            B.w0a = L.add.w0;
+            B.add = L.add.umac;
             for (int q = 0; q < 13; ++q) B.ks[q] = 8 * views[q]->ks;
             for (int q = 0; q < 9; ++q)
                 if (views[q]->js > lim || views[q]->ks > lim || views[q]->ns > lim)
@@ -1665,7 +1676,8 @@ int vp_launch(mx_adv_ctx* c, const std::vector<VFBox>& boxes, int tz, bool one_l
 
 }  // namespace
 
-int velpred_fused(mx_adv_ctx* c, const std::vector<VpLevel>& levs) {
+int velpred_fused(mx_adv_ctx* c, const std::vector<VpLevel>& levs, bool* added) {
+    if (added) *added = false;
     if (levs.empty()) return MX_OK;
     int rc = check_phys(c);
     if (rc) return rc;
@@ -1684,6 +1696,7 @@ int velpred_fused(mx_adv_ctx* c, const std::vector<VpLevel>& levs) {
     // (256 VGPRs); one component per block: the tile shape (cell columns)
     // and register budget (waves per SIMD) of `velpred_fused_tile`
     if (!c->vp_fused_comp || !rows) return vf_launch<16, 11, 2>(c, boxes, tz > 0 ? tz : 32, levs[0].lev);
+    if (added) *added = true;
     const bool one = levs.size() == 1;
     // 16 x 11 columns: ppm_type 1 at 4 waves per SIMD (1.20 ms per 256^3 launch
     // against 1.21 at 3), ppm_type 2 at 3, where 4 spill 67 VGPRs (1.72 against
