@@ -420,6 +420,14 @@ int velpred_setup(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_mu
                   const W0Add& add = {});
 int utrans_from_plan(mx_adv_ctx* c, const VpPlan& plan, bool fill = true);
 int velpred_finish(mx_adv_ctx* c, const VpPlan& plan);
+// MakeEdgeScal of listed components by the staged kernels, and the workspace
+// that their temporaries take
+size_t edge_ws_bytes(const mx_adv_ctx* c, int lev, int num_comp);
+int make_edge_scal_staged(mx_adv_ctx* c, int lev, const mx_multifab* state,
+                          const mx_face_multifab* sedge, const mx_face_multifab* umac,
+                          const mx_multifab* force, int is_vel, const mx_bcrec* bcs,
+                          const std::vector<int>& scomps, const std::vector<int>& bccomps,
+                          int is_conservative);
 int make_edge_scal(mx_adv_ctx* c, int lev, const mx_multifab* state,
                    const mx_face_multifab* sedge, const mx_face_multifab* umac,
                    const mx_multifab* force, int is_vel, const mx_bcrec* bcs, int nbccomp,

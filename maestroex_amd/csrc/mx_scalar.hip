@@ -34,10 +34,11 @@ struct EsTmp {
     DA Ip, Im, Ipf, Imf;  // ppm_type 0: Ip holds the slope along each direction
     DA T[6];
     int bclo[3], bchi[3];  // bcs[bccomp] of this component
+    int comp;              // the state / edge-state component
+    int pad_ = 0;          // explicit, so that equal tables are equal byte for byte
 };
 
 struct EsArgs {
-    int start_scomp;
     int num_comp;
     int is_vel;
     int is_conservative;
@@ -46,7 +47,7 @@ struct EsArgs {
 template <int PPM, int D>
 __device__ __forceinline__ void es_ppm_dir(const EsBox& B, const EsTmp& Tm, const KGeom& g,
                                            const EsArgs& A, int vc, int i, int j, int k) {
-    const int comp = A.start_scomp + vc;
+    const int comp = Tm.comp;
     const int pos = D == 0 ? i : (D == 1 ? j : k);
     const int bclo = Tm.bclo[D], bchi = Tm.bchi[D];
     double v[9];
@@ -96,7 +97,7 @@ template <int D>
 __device__ __forceinline__ void es_pred(const EsBox& B, const EsTmp& Tm, const KGeom& g,
                                         const EsArgs& A, int vc, int i, int j, int k, double& l,
                                         double& r) {
-    const int comp = A.start_scomp + vc;
+    const int comp = Tm.comp;
     const int im = i - e(D, 0), jm = j - e(D, 1), km = k - e(D, 2);
     if (g.ppm_type == 0) {
         const double u = B.um[D](i, j, k);
@@ -168,7 +169,7 @@ __device__ __forceinline__ double es_divu(const EsBox& B, const KGeom& g, int i,
 template <int D, int T>
 __device__ __forceinline__ void es_trans(const EsBox& B, const EsTmp& Tm, const KGeom& g,
                                          const EsArgs& A, int vc, int i, int j, int k) {
-    const int comp = A.start_scomp + vc;
+    const int comp = Tm.comp;
     const int im = i - e(D, 0), jm = j - e(D, 1), km = k - e(D, 2);
     const int it = e(T, 0), jt = e(T, 1), kt = e(T, 2);
     const double ht = g.dx[T];
@@ -299,7 +300,7 @@ __device__ __forceinline__ void es_edge_term(const EsBox& B, const EsTmp& Tm, co
 template <int D>
 __device__ __forceinline__ void es_edge(const EsBox& B, const EsTmp& Tm, const KGeom& g,
                                         const EsArgs& A, int vc, int i, int j, int k) {
-    const int comp = A.start_scomp + vc;
+    const int comp = Tm.comp;
     const int im = i - e(D, 0), jm = j - e(D, 1), km = k - e(D, 2);
     const double dt2 = 0.5 * g.dt;
     double fl, fr;
@@ -640,16 +641,39 @@ int make_edge_scal(mx_adv_ctx* c, int lev, const mx_multifab* state,
         fused_edge_rows_ok({lev, state, sedge, umac, force}))
         return make_edge_scal_fused(c, lev, state, sedge, umac, force, is_vel, bcs, start_scomp,
                                     start_bccomp, num_comp, is_conservative);
+    std::vector<int> sc, bc;
+    for (int n = 0; n < num_comp; ++n) {
+        sc.push_back(start_scomp + n);
+        bc.push_back(start_bccomp + n);
+    }
+    return make_edge_scal_staged(c, lev, state, sedge, umac, force, is_vel, bcs, sc, bc,
+                                 is_conservative);
+}
+
+size_t edge_ws_bytes(const mx_adv_ctx* c, int lev, int num_comp) {
+    const int dim = c->p.dim;
+    const auto& grids = c->grids[lev];
+    const bool tf = c->p.ppm_trace_forces == 1 && c->p.ppm_type != 0;
+    auto grown1 = [&](HBox b) { return grow(b, dim, 1); };
+    size_t need = (size_t)num_comp * 2 * tmp_bytes(grids, dim, grown1);
+    if (tf) need += (size_t)num_comp * 2 * tmp_bytes(grids, dim, grown1);
+    if (dim == 3) need += (size_t)num_comp * 6 * tmp_bytes(grids, 1, grown1);
+    return need;
+}
+
+int make_edge_scal_staged(mx_adv_ctx* c, int lev, const mx_multifab* state,
+                          const mx_face_multifab* sedge, const mx_face_multifab* umac,
+                          const mx_multifab* force, int is_vel, const mx_bcrec* bcs,
+                          const std::vector<int>& scomps, const std::vector<int>& bccomps,
+                          int is_conservative) {
+    const int num_comp = (int)scomps.size();
     const int dim = c->p.dim;
     const auto& grids = c->grids[lev];
     const int ppm = c->p.ppm_type;
     const bool tf = c->p.ppm_trace_forces == 1 && ppm != 0;
     auto grown1 = [&](HBox b) { return grow(b, dim, 1); };
 
-    size_t need = (size_t)num_comp * 2 * tmp_bytes(grids, dim, grown1);
-    if (tf) need += (size_t)num_comp * 2 * tmp_bytes(grids, dim, grown1);
-    if (dim == 3) need += (size_t)num_comp * 6 * tmp_bytes(grids, 1, grown1);
-    int rc = ws_reserve(c, need);
+    int rc = ws_reserve(c, edge_ws_bytes(c, lev, num_comp));
     if (rc) return rc;
 
     std::vector<EsTmp> tmps(grids.size() * num_comp);
@@ -671,9 +695,10 @@ int make_edge_scal(mx_adv_ctx* c, int lev, const mx_multifab* state,
             t.Imf = tf ? Imf[b] : null_da();
             for (int p = 0; p < 6; ++p) t.T[p] = dim == 3 ? T[p][b] : null_da();
             for (int d = 0; d < 3; ++d) {
-                t.bclo[d] = bcs[start_bccomp + vc].lo[d];
-                t.bchi[d] = bcs[start_bccomp + vc].hi[d];
+                t.bclo[d] = bcs[bccomps[vc]].lo[d];
+                t.bchi[d] = bcs[bccomps[vc]].hi[d];
             }
+            t.comp = scomps[vc];
         }
     }
     std::vector<EsBox> boxes;
@@ -696,7 +721,6 @@ int make_edge_scal(mx_adv_ctx* c, int lev, const mx_multifab* state,
     }
     EsArgs A;
     std::memset(&A, 0, sizeof(A));
-    A.start_scomp = start_scomp;
     A.num_comp = num_comp;
     A.is_vel = is_vel;
     A.is_conservative = is_conservative;
@@ -1086,11 +1110,27 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
             for (int n = 0; n < gr[1]; ++n) sc.push_back(gr[0] + n);
         if ((rc = make_edge_scal_fused_list(c, levs, 0, bs, sc, sc, 0))) return rc;
     } else {
-        for (int i = 0; i < nlev; ++i)
+        // the staged kernels take the three calls in one, too, where the calls'
+        // own launches count (four of the 16 of a 2-D pass, 256^2: 103 -> 88 us)
+        // and the temporaries of all their components at once are small; the
+        // fixed scratch of the allocation-free pass holds one call's
+        std::vector<int> all;
+        for (const auto& gr : groups)
+            for (int n = 0; n < gr[1]; ++n) all.push_back(gr[0] + n);
+        constexpr size_t kOneCall = (size_t)128 << 20;
+        for (int i = 0; i < nlev; ++i) {
+            const bool own = fused_edge_scal_ok(c, 0);  // a call's own choice, by its rows
+            if (!own && !c->ext_ws && edge_ws_bytes(c, lev0 + i, (int)all.size()) <= kOneCall) {
+                if ((rc = make_edge_scal_staged(c, lev0 + i, &a[i].scal, &a[i].sedge, &a[i].umac,
+                                                &a[i].scal_force, 0, bs, all, all, 0)))
+                    return rc;
+                continue;
+            }
             for (const auto& gr : groups)
                 if ((rc = make_edge_scal(c, lev0 + i, &a[i].scal, &a[i].sedge, &a[i].umac,
                                          &a[i].scal_force, 0, bs, nbs, gr[0], gr[0], gr[1], 0)))
                     return rc;
+        }
     }
     for (int i = 0; i < nlev; ++i) {
         const int lev = lev0 + i;

@@ -43,6 +43,7 @@ struct UtBox {
 
 struct UtArgs {
     int bclo[3][3], bchi[3][3];  // bcs_u[comp].lo/hi[dir]
+    DivBy h[3];                  // the cell widths
 };
 
 // Addw0 of a D-face where it is stored (a pass of its own reads and writes the
@@ -236,7 +237,8 @@ __device__ __forceinline__ void utrans_rows(const UtBox& B, const KGeom& g, cons
         load_stencil<PPM>(B.ut.p + B.ut.off(i, j, k, 0), 1, v);
         ppm_edges<PPM, 0>(v, i, g.domlo[0], g.domhi[0], A.bclo[0][0], A.bchi[0][0], sm, sp);
         const double uc = B.uf(i, j, k, 0);
-        ppm_trace(v[4], sm, sp, uc, uc, g.dt, g.dx[0], g.rel_eps, Ip, Im);
+        const double sig = div_by(dabs(uc) * g.dt, A.h[0]);
+        trace_sig(v[4], sm, sp, uc, uc, sig, sig, g.rel_eps, Ip, Im);
     }
     // every lane takes part in the shuffle; lane 0's result is unused
     const double Ipl = __shfl_up(Ip, 1u, 64);
@@ -312,7 +314,8 @@ __device__ __forceinline__ void utrans_march(const UtBox& B, const KGeom& g, con
         if (ppm_special<PPM>(cpos, dlo, dhi, bclo, bchi))
             ppm_edges<PPM, D>(v, cpos, dlo, dhi, bclo, bchi, sm, sp);
         if (PPM == 1) zf0 = zf1;
-        ppm_trace(v[4], sm, sp, uc, uc, g.dt, g.dx[D], g.rel_eps, Ip, Im);
+        const double sig = div_by(dabs(uc) * g.dt, A.h[D]);
+        trace_sig(v[4], sm, sp, uc, uc, sig, sig, g.rel_eps, Ip, Im);
         if (cpos >= f0) {
             const int j = D == 1 ? cpos : tt, k = D == 2 ? cpos : tt;
             double x = utrans_riemann<D>(B, g, i, j, k, Ipl, Im);
@@ -898,6 +901,7 @@ int make_utrans(mx_adv_ctx* c, int lev, const mx_multifab* utilde, const mx_mult
             lblocks = std::max(lblocks, (n0 * std::max(n1, n2) * nch + UT_NT - 1) / UT_NT);
         }
     UtArgs A;
+    for (int d = 0; d < 3; ++d) A.h[d] = div_const(c->p.dx[lev][d]);
     for (int n = 0; n < 3; ++n)
         for (int d = 0; d < 3; ++d) {
             A.bclo[n][d] = c->bcs_u[n].lo[d];
