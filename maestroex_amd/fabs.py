@@ -6,7 +6,8 @@ order -- and described to the C-ABI by an `mx_fab` (maestroex_amd._abi.Fab).
 Face-centred data ("nodal" in one direction) have one more point in that
 direction, as in AMReX.  2-D data use nz == 1 and k == 0.
 """
-import ctypes as C
+import ctypes
+import struct
 
 import numpy as np
 
@@ -53,6 +54,11 @@ def split_domain(geom, max_grid):
             for ix in ranges[0]:
                 boxes.append(((ix[0], jy[0], kz[0]), (ix[1], jy[1], kz[1])))
     return boxes
+
+
+# _abi.Fab's layout
+_FAB = struct.Struct("@Pqqq7i4x")
+assert _FAB.size == ctypes.sizeof(_abi.Fab)
 
 
 class Backend:
@@ -117,29 +123,23 @@ class MultiFab:
             self.begin.append(b)
         self._desc = None
 
-    def fab_desc(self, b):
+    def _pack(self, b):
+        """The bytes of box b's descriptor (_abi.Fab).  Packed, not set field by
+        field: a pass describes some 15 MultiFabs per call, which took more time
+        than its launches on one small box."""
         a = self.arrays[b]
-        beg = self.begin[b]
+        x, y, z = self.begin[b]
         nc, nz, ny, nx = a.shape
-        f = _abi.Fab()
-        f.p = self.backend.ptr(a)
-        f.jstride = nx
-        f.kstride = nx * ny
-        f.nstride = nx * ny * nz
-        for d in range(3):
-            f.begin[d] = beg[d]
-        f.end[0] = beg[0] + nx
-        f.end[1] = beg[1] + ny
-        f.end[2] = beg[2] + nz
-        f.ncomp = nc
-        return f
+        return _FAB.pack(self.backend.ptr(a), nx, nx * ny, nx * ny * nz, x, y, z, x + nx, y + ny,
+                         z + nz, nc)
+
+    def fab_desc(self, b):
+        return _abi.Fab.from_buffer_copy(self._pack(b))
 
     def desc(self):
         n = len(self.arrays)
-        fabs = (_abi.Fab * n)(*[self.fab_desc(b) for b in range(n)])
-        m = _abi.MultiFabDesc()
-        m.nfab = n
-        m.fab = C.cast(fabs, C.POINTER(_abi.Fab))
+        fabs = (_abi.Fab * n).from_buffer_copy(b"".join([self._pack(b) for b in range(n)]))
+        m = _abi.MultiFabDesc(n, fabs)
         m._keep = fabs
         return m
 
@@ -192,12 +192,8 @@ class FaceMultiFab:
         return self.d[d]
 
     def desc(self):
-        f = _abi.FaceMultiFabDesc()
-        keep = []
-        for d in range(self.dim):
-            m = self.d[d].desc()
-            keep.append(m)
-            f.dir[d] = m
+        keep = [self.d[d].desc() for d in range(self.dim)]
+        f = _abi.FaceMultiFabDesc(tuple(keep))
         f._keep = keep
         return f
 
@@ -220,11 +216,7 @@ class BaseState:
         self.array = backend.from_numpy(data)
 
     def desc(self):
-        s = _abi.BaseStateDesc()
-        s.p = self.backend.ptr(self.array)
-        s.nlev = self.nlev
-        s.len = self.len
-        return s
+        return _abi.BaseStateDesc(self.backend.ptr(self.array), self.nlev, self.len)
 
     def to_numpy(self):
         return np.array(self.backend.to_numpy(self.array))
