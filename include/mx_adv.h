@@ -248,7 +248,8 @@ int mx_adv_prof_read(mx_adv_ctx* ctx, int idx, const char** name, double* total_
                         1.
      "adjoint_face_sums", "adjoint_state_fused", "adjoint_pow2_index",
      "adjoint_trace_rolled", "adjoint_xcd"  arrangements of the step
-                        adjoint's kernels (defaults 0, 1, 1, 0, 0); every
+                        adjoint's kernels (defaults 0, 1, 1, 0 and, for the
+                        last, 1 over box lists, 0 on one periodic box); every
                         choice gives bit-identical results.
    Unknown keys and out-of-range values return MX_ERR_ARG. */
 int mx_adv_set_tuning(mx_adv_ctx* ctx, const char* key, long long value);

@@ -1779,7 +1779,7 @@ int mx_adv_scal_step_vjp(mx_adv_ctx* c, mx_fab* s, mx_fab* umac, const mx_fab* g
     for (int d = 0; d < 3; ++d) A.ext[d] = n;
     ab_factors(c, A, ncomp);
 
-    A.xcd = c->adj_xcd;
+    A.xcd = c->adj_xcd == 1;
     dim3 g1 = grid1(n3);
     if (A.xcd) g1.x = (g1.x + 7u) & ~7u;
     const dim3 gc(g1.x, (unsigned)ncomp);
@@ -2050,7 +2050,7 @@ int mx_adv_scal_step_vjp_boxes(mx_adv_ctx* c, const mx_multifab* s, const mx_fac
                   A.ext[2], L.pad[0], L.pad[1], L.pad[2]);
     std::memcpy(c->adj_layout, layout, sizeof(layout));
 
-    A.xcd = c->adj_xcd;
+    A.xcd = c->adj_xcd != 0;
     dim3 g1 = grid1(npt);
     if (A.xcd) g1.x = (g1.x + 7u) & ~7u;
     const dim3 gc(g1.x, (unsigned)ncomp);
