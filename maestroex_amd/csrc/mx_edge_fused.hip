@@ -574,7 +574,10 @@ __global__ void __launch_bounds__(fused_nt(TX, TY))
                 sz = pz ? t : s0;
                 zf0 = zf1;
                 zf1 = zf2;
-                if (z_general(q)) {
+                // (face z0 - 1 enters nothing that is stored, and its low cell's
+                // stencil would reach a plane past the ghosts of a box that
+                // starts two or three planes above the domain's low side)
+                if (q >= z0 && z_general(q)) {
                     cbox* Bf = fresh(&B);
                     const int dl = Bf->domlo[2], dh = Bf->domhi[2];
                     const int pos = q - (fz.left ? 1 : 0);
