@@ -1112,15 +1112,16 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
     } else {
         // the staged kernels take the three calls in one, too, where the calls'
         // own launches count (four of the 16 of a 2-D pass, 256^2: 103 -> 88 us)
-        // and the temporaries of all their components at once are small; the
-        // fixed scratch of the allocation-free pass holds one call's
+        // and the temporaries of all their components at once are small (half of
+        // the allocation-free pass's scratch, whose sizing run and whose run must
+        // choose alike)
         std::vector<int> all;
         for (const auto& gr : groups)
             for (int n = 0; n < gr[1]; ++n) all.push_back(gr[0] + n);
         constexpr size_t kOneCall = (size_t)128 << 20;
         for (int i = 0; i < nlev; ++i) {
             const bool own = fused_edge_scal_ok(c, 0);  // a call's own choice, by its rows
-            if (!own && !c->ext_ws && edge_ws_bytes(c, lev0 + i, (int)all.size()) <= kOneCall) {
+            if (!own && edge_ws_bytes(c, lev0 + i, (int)all.size()) <= kOneCall) {
                 if ((rc = make_edge_scal_staged(c, lev0 + i, &a[i].scal, &a[i].sedge, &a[i].umac,
                                                 &a[i].scal_force, 0, bs, all, all, 0)))
                     return rc;
