@@ -771,14 +771,17 @@ bool fused_edge_scal_ok(const mx_adv_ctx* c, int is_conservative) {
            c->p.ppm_trace_forces == 0 && c->fused_edge;
 }
 
-// a tile and its stencil span at most 25 rows (32-bit byte offsets in a plane)
+// unsigned 32-bit byte offsets in a plane: a tile and its stencil span at most 25
+// rows, which follow each other upwards
 bool fused_edge_rows_ok(const EdgeLevel& L) {
     const long long lim = 0x7fffffffLL / (8 * 26);
     const long long max = 0x7fffffffLL;  // past which the launch refuses them
     auto ok = [&](const mx_multifab* m) {
-        for (int b = 0; b < m->nfab; ++b)
-            if (m->fab[b].jstride > lim && m->fab[b].jstride <= max && m->fab[b].kstride <= max)
-                return false;
+        for (int b = 0; b < m->nfab; ++b) {
+            const long long js = m->fab[b].jstride;
+            if (js > max || m->fab[b].kstride > max) continue;
+            if (js < 0 || js > lim) return false;
+        }
         return true;
     };
     bool r = ok(L.state) && ok(L.force);

@@ -1684,13 +1684,13 @@ int velpred_fused(mx_adv_ctx* c, const std::vector<VpLevel>& levs, bool* added) 
     std::vector<VFBox> boxes;
     if ((rc = vf_boxes(c, levs, boxes))) return rc;
     const int tz = c->vp_fused_tz;
-    // rows past the per-component kernel's 32-bit byte offsets (a tile and its
-    // stencil span at most 25 rows)
+    // rows past the per-component kernel's unsigned 32-bit byte offsets (a tile
+    // and its stencil span at most 25 rows), or that run downwards
     bool rows = true;
     for (const VFBox& B : boxes) {
         const DA* views[] = {&B.ut,    &B.fo,    &B.uf,     &B.tr[0],  &B.tr[1],  &B.tr[2], &B.um[0],
                              &B.um[1], &B.um[2], &B.w0m[0], &B.w0m[1], &B.w0m[2], &B.w0c};
-        for (const DA* d : views) rows = rows && d->js <= 0x7fffffffLL / (8 * 26);
+        for (const DA* d : views) rows = rows && d->js >= 0 && d->js <= 0x7fffffffLL / (8 * 26);
     }
     // all three components per block: 16 x 11 columns at 2 waves per SIMD
     // (256 VGPRs); one component per block: the tile shape (cell columns)
