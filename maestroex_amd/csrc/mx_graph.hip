@@ -270,6 +270,10 @@ int mx_adv_autotune(mx_adv_ctx* c, int nlev, const mx_adv_pass_args* args,
     std::vector<EdgeLevel> levs;
     for (int i = 0; i < nlev; ++i)
         levs.push_back({i, &args[i].scal, &args[i].sedge, &args[i].umac, &args[i].scal_force});
+    // the pass takes the staged kernels for FABs whose rows the fused one cannot
+    // address
+    for (const EdgeLevel& L : levs)
+        if (!fused_edge_rows_ok(L)) return MX_ERR_UNSUPPORTED;
     const mx_bcrec* bs = c->bcs_s.data();
     const int tiles[] = {4, 2, 3, 0};
     const int tzs[] = {16, 32, 64, 128};

@@ -1,11 +1,11 @@
 """GPU parity of the pass over FABs whose rows do not follow each other at nx doubles:
 rows far apart (past the fused kernels' 32-bit byte offsets: the row index is the
 slowest, so that the FAB stays small) and rows that run downwards.  Against the CPU
-oracle, bit for bit."""
-import numpy as np
+oracle, bit for bit; the autotuner of the fused kernel refuses such levels."""
 import pytest
 
 from harness import assert_bitexact, compare_face, gpu_for, oracle_for, pair
+from maestroex_amd import _abi
 from maestroex_amd.fabs import _FAB
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +50,14 @@ def test_pass_row_strides(ppm, field, far):
     for name in ("utrans", "umac", "sedge", "sflux"):
         comps = None if name in ("utrans", "umac") else [0, 1] + list(range(4, wc.nscal))
         assert_bitexact(compare_face(getattr(wc, name), getattr(wg, name), comps=comps), name)
+
+
+@pytest.mark.parametrize("far", [True, False], ids=["far", "down"])
+def test_autotune_refuses(far):
+    _, wg = pair(dim=3, n=8, max_grid=8, ppm_type=1)
+    restride(wg.sedge[0], far)
+    m = gpu_for(wg)
+    with pytest.raises(_abi.MxError) as e:
+        m.autotune([wg.pass_fields()])
+    assert e.value.code == _abi.MX_ERR_UNSUPPORTED
+    m.sync()
