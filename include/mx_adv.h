@@ -462,14 +462,15 @@ int mx_adv_pass_graph_destroy(mx_adv_graph* g);
 
 /* Autotuner of the fused edge-state kernel (no counterpart in the
    reference): runs the hierarchy pass once, then times the species edge-state
-   launch for every tile shape (16x11, 16x12, 16x8, 32x8 columns) and z-chunk (16,
-   32, 64, 128 planes), keeps the fastest in the context ("edge_scal_tile",
-   "edge_scal_tz") and reports every candidate. */
+   launch for every tile shape (16x11, 16x12, 16x8, 32x8 columns) and z-chunk (as
+   the launch picks it, reported as tz 0, and 16, 64, 128 planes), keeps the fastest
+   in the context ("edge_scal_tile", "edge_scal_tz") and reports every candidate.
+   MX_ERR_UNSUPPORTED where the pass does not take that kernel. */
 #define MX_TUNE_MAX 16
 typedef struct {
     int ncand;
     int tile[MX_TUNE_MAX];
-    int tz[MX_TUNE_MAX];
+    int tz[MX_TUNE_MAX]; /* planes per chunk; 0: picked by the launch */
     double ms[MX_TUNE_MAX];
     int best; /* index of the chosen candidate */
 } mx_adv_tune_report;

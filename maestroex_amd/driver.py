@@ -396,7 +396,8 @@ class Maestro:
 
     def autotune(self, fields):
         """Pick the fused edge kernel's tile shape and z-chunk; returns the
-        candidates as a list of (tile, tz, ms) and the chosen index."""
+        candidates as a list of (tile, tz, ms), tz 0 for chunks that the launch
+        picks, and the chosen index."""
         arr, keep = self._levels_args(fields)
         rep = _abi.TuneReport()
         self._check(self.fns["autotune"](self.ctx, len(fields), arr, C.byref(rep)), "autotune")
