@@ -251,7 +251,10 @@ int mx_adv_prof_read(mx_adv_ctx* ctx, int idx, const char** name, double* total_
                         adjoint's kernels (defaults 0, 1, 1, 0 and, for the
                         last, 1 over box lists, 0 on one periodic box); every
                         choice gives bit-identical results.
-   Unknown keys and out-of-range values return MX_ERR_ARG. */
+   MX_TUNE_DEFAULT returns a key to what a new context has, also where that is a
+   choice made per launch ("unset" above).  Unknown keys and out-of-range values
+   return MX_ERR_ARG. */
+#define MX_TUNE_DEFAULT (-0x7fffffffffffffffLL - 1)
 int mx_adv_set_tuning(mx_adv_ctx* ctx, const char* key, long long value);
 
 /* ---- unit-level kernels ------------------------------------------------- */

@@ -250,6 +250,7 @@ SIGNATURES = {
 }
 
 MX_TUNE_MAX = 16
+MX_TUNE_DEFAULT = -2**63
 
 
 class TuneReport(C.Structure):

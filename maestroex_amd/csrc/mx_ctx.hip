@@ -5,6 +5,7 @@
 #include <cmath>
 #include <array>
 #include <cstdio>
+#include <cstring>
 
 #include "mx_internal.H"
 
@@ -894,74 +895,45 @@ int mx_adv_prof_enable(mx_adv_ctx* c, int on) {
 
 int mx_adv_set_tuning(mx_adv_ctx* c, const char* key, long long value) {
     if (!c || !key) return MX_ERR_ARG;
-    const std::string k(key);
-    if (k == "edge_scal_fused") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->fused_edge = (int)value;
-    } else if (k == "edge_scal_tz") {
-        if (value < 1 || value > 4096) return MX_ERR_ARG;
-        c->fused_tz = (int)value;
-    } else if (k == "edge_scal_tile") {
-        if (value < -1 || value > 4) return MX_ERR_ARG;
-        c->fused_tile = (int)value;
-    } else if (k == "edge_scal_per_box") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->fused_per_box = (int)value;
-    } else if (k == "utrans_line") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->utrans_line = (int)value;
-    } else if (k == "utrans_chunks") {
-        if (value < 1 || value > 64) return MX_ERR_ARG;
-        c->utrans_chunks = (int)value;
-    } else if (k == "velpred_trans_all") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->vp_trans_all = (int)value;
-    } else if (k == "velpred_ppm_all") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->vp_ppm_all = (int)value;
-    } else if (k == "velpred_fused") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->vp_fused = (int)value;
-    } else if (k == "rhoh_flux_epilogue") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->rhoh_flux_epilogue = (int)value;
-    } else if (k == "velpred_fused_comp") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->vp_fused_comp = (int)value;
-    } else if (k == "velpred_fused_tile") {
-        if (value < 0 || value > 5) return MX_ERR_ARG;
-        c->vp_fused_tile = (int)value;
-    } else if (k == "velpred_fused_tz") {
-        if (value < 1 || value > 4096) return MX_ERR_ARG;
-        c->vp_fused_tz = (int)value;
-    } else if (k == "xcd_remap") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->xcd_remap = (int)value;
-    } else if (k == "adjoint_state_fused") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->adj_state_fused = (int)value;
-    } else if (k == "adjoint_face_sums") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->adj_face_sums = (int)value;
-    } else if (k == "velpred_fused_xcd") {
-        if (value < -1 || value > 2) return MX_ERR_ARG;
-        c->vp_fused_xcd = (int)value;
-    } else if (k == "edge_scal_xcd") {
-        if (value < 0 || value > 2) return MX_ERR_ARG;
-        c->es_fused_xcd = (int)value;
-    } else if (k == "adjoint_xcd") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->adj_xcd = (int)value;
-    } else if (k == "adjoint_trace_rolled") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->adj_trace_rolled = (int)value;
-    } else if (k == "adjoint_pow2_index") {
-        if (value != 0 && value != 1) return MX_ERR_ARG;
-        c->adj_pow2 = (int)value;
-    } else {
-        return MX_ERR_ARG;
+    struct Key {
+        const char* name;
+        int mx_adv_ctx::*field;
+        int lo, hi;
+    };
+    static const Key keys[] = {
+        {"edge_scal_fused", &mx_adv_ctx::fused_edge, 0, 1},
+        {"edge_scal_tz", &mx_adv_ctx::fused_tz, 1, 4096},
+        {"edge_scal_tile", &mx_adv_ctx::fused_tile, -1, 4},
+        {"edge_scal_per_box", &mx_adv_ctx::fused_per_box, 0, 1},
+        {"edge_scal_xcd", &mx_adv_ctx::es_fused_xcd, 0, 2},
+        {"utrans_line", &mx_adv_ctx::utrans_line, 0, 1},
+        {"utrans_chunks", &mx_adv_ctx::utrans_chunks, 1, 64},
+        {"velpred_trans_all", &mx_adv_ctx::vp_trans_all, 0, 1},
+        {"velpred_ppm_all", &mx_adv_ctx::vp_ppm_all, 0, 1},
+        {"velpred_fused", &mx_adv_ctx::vp_fused, 0, 1},
+        {"velpred_fused_comp", &mx_adv_ctx::vp_fused_comp, 0, 1},
+        {"velpred_fused_tile", &mx_adv_ctx::vp_fused_tile, 0, 5},
+        {"velpred_fused_tz", &mx_adv_ctx::vp_fused_tz, 1, 4096},
+        {"velpred_fused_xcd", &mx_adv_ctx::vp_fused_xcd, -1, 2},
+        {"rhoh_flux_epilogue", &mx_adv_ctx::rhoh_flux_epilogue, 0, 1},
+        {"xcd_remap", &mx_adv_ctx::xcd_remap, 0, 1},
+        {"adjoint_state_fused", &mx_adv_ctx::adj_state_fused, 0, 1},
+        {"adjoint_face_sums", &mx_adv_ctx::adj_face_sums, 0, 1},
+        {"adjoint_xcd", &mx_adv_ctx::adj_xcd, 0, 1},
+        {"adjoint_trace_rolled", &mx_adv_ctx::adj_trace_rolled, 0, 1},
+        {"adjoint_pow2_index", &mx_adv_ctx::adj_pow2, 0, 1},
+    };
+    for (const Key& k : keys) {
+        if (std::strcmp(k.name, key) != 0) continue;
+        if (value == MX_TUNE_DEFAULT) {
+            c->*k.field = mx_adv_ctx().*k.field;
+            return MX_OK;
+        }
+        if (value < k.lo || value > k.hi) return MX_ERR_ARG;
+        c->*k.field = (int)value;
+        return MX_OK;
     }
-    return MX_OK;
+    return MX_ERR_ARG;
 }
 
 int mx_adv_prof_read(mx_adv_ctx* c, int idx, const char** name, double* total_ms,

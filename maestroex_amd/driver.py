@@ -68,8 +68,10 @@ class Maestro:
         return bs, bu
 
     def set_tuning(self, key, value):
-        """Kernel selection / launch shape; results are identical for every choice."""
-        self._check(self.fns["set_tuning"](self.ctx, key.encode(), int(value)), "set_tuning")
+        """Kernel selection / launch shape; results are identical for every choice.
+        value None: the key's default."""
+        value = _abi.MX_TUNE_DEFAULT if value is None else int(value)
+        self._check(self.fns["set_tuning"](self.ctx, key.encode(), value), "set_tuning")
 
     def sync(self):
         if "sync" in self.fns:
