@@ -837,12 +837,12 @@ int launch_one(mx_adv_ctx* c, const FBox* db, const FTile* dtl, size_t ntile, co
     return MX_OK;
 }
 
-// blocks of the open-boundary kernel a CU holds
-template <int PPM, bool CONS, int TX, int TY>
+// blocks of the kernel a CU holds
+template <int PPM, bool CONS, int TX, int TY, int MODE>
 int fused_blocks() {
     static const int n = [] {
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_es_fused<PPM, CONS, TX, TY, 0>,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_es_fused<PPM, CONS, TX, TY, MODE>,
                                                          fused_nt(TX, TY), 0) != hipSuccess) {
             (void)hipGetLastError();
             v = 0;
@@ -850,6 +850,12 @@ int fused_blocks() {
         return v > 0 ? v : 3;
     }();
     return n;
+}
+template <int TX, int TY, int MODE>
+int fused_blocks(int ppm, bool cons) {
+    if (ppm == 1)
+        return cons ? fused_blocks<1, true, TX, TY, MODE>() : fused_blocks<1, false, TX, TY, MODE>();
+    return cons ? fused_blocks<2, true, TX, TY, MODE>() : fused_blocks<2, false, TX, TY, MODE>();
 }
 
 template <int TX, int TY>
@@ -912,13 +918,15 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
                                     ? 0
                                     : 1];
             cols.push_back(col);
+            zgen = zgen || (col.tiles[0] && !tile_clear(g.lo[2], col.nz, B.domlo[2], B.domhi[2],
+                                                        act[2][0], act[2][1]));
         }
     }
     if (tz <= 0) {
-        const int per_cu = c->p.ppm_type == 1
-                               ? (cons ? fused_blocks<1, true, TX, TY>() : fused_blocks<1, false, TX, TY>())
-                               : (cons ? fused_blocks<2, true, TX, TY>() : fused_blocks<2, false, TX, TY>());
-        const int blocks[2] = {per_cu, std::min(per_cu, 3)};
+        // of the two launches' kernels
+        const int blocks[2] = {zgen ? fused_blocks<TX, TY, 1>(c->p.ppm_type, cons)
+                                    : fused_blocks<TX, TY, 0>(c->p.ppm_type, cons),
+                               fused_blocks<TX, TY, 2>(c->p.ppm_type, cons)};
         tz = pick_chunks(cols, num_comp, blocks);
     }
     for (size_t id = 0; id < boxes.size(); ++id) {
@@ -943,7 +951,6 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
                                         s == 1 && act[2][1]))
                             T.zgen |= 1 << s;
                     (f ? tiles : btiles).push_back(T);
-                    zgen = zgen || (f && T.zgen);
                 }
     }
     const size_t nfree = tiles.size();

@@ -1560,19 +1560,24 @@ int vf_launch(mx_adv_ctx* c, const std::vector<VFBox>& boxes, int tz, int lev) {
     return rc ? rc : launch(std::false_type{}, dt + nfree, tiles.size() - nfree);
 }
 
-// blocks of the open-boundary kernel a CU holds
-template <int PPM, int TX, int TY, int WPE>
+// blocks of the kernel a CU holds; WPE as in vp_launch
+template <int PPM, int TX, int TY, int MODE, int WPE>
 int vp_blocks() {
+    constexpr int W = MODE == 0 ? WPE : 3;
     static const int n = [] {
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_vp_fused_comp<PPM, TX, TY, 0, WPE>,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_vp_fused_comp<PPM, TX, TY, MODE, W>,
                                                          vf_nt(TX, TY), 0) != hipSuccess) {
             (void)hipGetLastError();
             v = 0;
         }
-        return v > 0 ? v : WPE;
+        return v > 0 ? v : W;
     }();
     return n;
+}
+template <int TX, int TY, int MODE, int WPE>
+int vp_blocks(int ppm) {
+    return ppm == 1 ? vp_blocks<1, TX, TY, MODE, WPE>() : vp_blocks<2, TX, TY, MODE, WPE>();
 }
 
 // one component per block.  WPE: the register budget (waves per SIMD) of the
@@ -1597,10 +1602,13 @@ int vp_launch(mx_adv_ctx* c, const std::vector<VFBox>& boxes, int tz, bool one_l
                                     ? 0
                                     : 1];
             cols.push_back(col);
+            zgen = zgen || (col.tiles[0] && !vf_tile_free(B.lo[2], col.nz, B.domlo[2], B.domhi[2],
+                                                          act[2][0], act[2][1]));
         }
-        const int per_cu =
-            c->p.ppm_type == 1 ? vp_blocks<1, TX, TY, WPE>() : vp_blocks<2, TX, TY, WPE>();
-        const int blocks[2] = {per_cu, std::min(per_cu, 3)};
+        // of the two launches' kernels
+        const int ppm = c->p.ppm_type;
+        const int blocks[2] = {zgen ? vp_blocks<TX, TY, 1, WPE>(ppm) : vp_blocks<TX, TY, 0, WPE>(ppm),
+                               vp_blocks<TX, TY, 2, WPE>(ppm)};
         tz = pick_chunks(cols, 3, blocks);
     }
     std::vector<VPTile> tiles, btiles;  // clear of general x/y sides, the others
