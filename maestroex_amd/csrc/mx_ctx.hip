@@ -18,12 +18,17 @@ namespace mxh {
 // need, its tables and first loads, its last edges).  A CU steps its resident
 // blocks together: n of the most it holds take a step in (0.86 + 0.14 n / most)
 // of the time of all of them (the edge kernel: 4.3 us alone, 4.8 us with 4).
-// Blocks past a full chip's take another round, and the rounds of a long
-// launch end raggedly (a quarter of a block).  So short chunks fill an idle
-// chip and even out the last round, and cost lead-in planes where there is work
-// for many rounds.  The edge kernel against chunks of 32 planes everywhere: one
-// 32^3 box 0.161 -> 0.031 ms (30 -> 480 blocks), 50^3 in 8 boxes 0.094 -> 0.051
-// ms, 256^3 unchanged; the best chunk of a sweep is 0 to 3% faster.
+// Blocks past a full chip's take another round, and a launch ends raggedly: a
+// quarter of a block after several rounds, a fifth after a single one (whose blocks
+// do not spread evenly over the CUs either).  So short chunks fill an idle chip and
+// even out the last round, and cost lead-in planes where there is work for many
+// rounds.
+// Against sweeps of 2 to 64 planes over 400 random box lists (edges 24 to 240, 1 to
+// 27 boxes, ppm_type 1 and 2, the edge kernel and VelPred), the pick is 1.7% from the
+// best length on average, more than 5% in 11% of the launches and 16% at worst
+// (3.1%, 21% and 32% when a single round was taken to end evenly).  Edge kernel
+// against 32 planes everywhere: one 32^3 box 0.160 -> 0.030 ms, 64^3 0.158 -> 0.084,
+// 96^3 0.241 -> 0.214, 256^3 in 8 boxes the same.
 int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, const int blocks_per_cu[2]) {
     constexpr int kCus = 256;
     static const int cand[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64};
@@ -47,7 +52,7 @@ int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, const int blocks_p
             const double full = std::floor(nb / slots);
             const double rem = std::ceil((nb - full * slots) / kCus);
             const double last = rem > 0.0 ? 0.86 + 0.14 * rem / blocks_per_cu[l] : 0.0;
-            t += full > 0.0 ? (full + last) * steps / nb + 0.25 * lmax : last * lmax;
+            t += full > 0.0 ? (full + last) * steps / nb + 0.25 * lmax : (last + 0.2) * lmax;
         }
         if (t < best_t * 0.995) {
             best_t = t;
@@ -56,7 +61,6 @@ int pick_chunks(const std::vector<ChunkCols>& cols, int nvar, const int blocks_p
     }
     return best;
 }
-
 
 KGeom kgeom(const mx_adv_ctx* c, int lev) {
     KGeom g;
