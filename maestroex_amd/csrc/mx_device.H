@@ -69,7 +69,9 @@ __device__ __forceinline__ double dsign1(double b) { return copysign(1.0, b); }
 // quotient, and one residual step from such a value gives the correctly
 // rounded quotient (Markstein, "Computation of elementary functions on the IBM
 // RISC System/6000", 1990).  div_fixup sets the results for x = 0, infinity and
-// NaN as the division does.  (Quotients below 2^-969 may round differently.)
+// NaN as the division does, and infinity for a quotient past the largest double,
+// whose residual step is NaN.  (The residual is exact for |x| >= 2^-969; below,
+// the quotient may round the other way: seen for |x| < 2^-1010.)
 struct DivBy {
     double d, r, rl;
 };
@@ -94,7 +96,7 @@ __device__ __forceinline__ double uniform(double x) {
     return v.d;
 }
 // x / 6: 1/6 rounded alone is enough, no quotient by 3 lies close to halfway
-// between two doubles
+// between two doubles (|x| < 2^-969 as above)
 __device__ __forceinline__ double div6(double x) {
     double q = x * (1.0 / 6.0);
     q = fma(fma(-6.0, q, x), 1.0 / 6.0, q);
