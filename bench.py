@@ -131,6 +131,11 @@ def committed_traffic(kernel, workload_tag):
     return None
 
 
+def tuned_shape(cand):
+    """The launch shape of an autotuner candidate (tile, tz, ms)."""
+    return {"tile": TILE_NAMES[cand[0]], "tz": cand[1] or "picked"}
+
+
 def host_cpu():
     """(nproc, CPU model name) of this host."""
     model = "unknown"
@@ -262,7 +267,7 @@ def amr_main(args, emit=True):
         key, val = kv.split("=")
         m.set_tuning(key, int(val))
     cands, best = m.autotune(fields)
-    tuned = {"tile": TILE_NAMES[cands[best][0]], "tz": cands[best][1]}
+    tuned = tuned_shape(cands[best])
     print(f"[bench] autotune {cands} -> {tuned}", file=sys.stderr, flush=True)
     eager_ms = time_ms(lambda: m.advance_pass_levels(fields), args.steps, args.warmup)
     g = m.pass_graph(fields)
@@ -354,8 +359,7 @@ def amr_main(args, emit=True):
                 "ns_per_cell": round(per_cell, 4),
                 "single_box_ns_per_cell": round(per_cell_1, 4),
                 "per_cell_ratio_vs_single_box": round(per_cell / per_cell_1, 4),
-                "single_box_autotuned": {"tile": TILE_NAMES[cands1[best1][0]],
-                                         "tz": cands1[best1][1]},
+                "single_box_autotuned": tuned_shape(cands1[best1]),
                 "autotuned": tuned,
                 "autotune_candidates_ms": [[c[0], c[1], round(c[2], 4)] for c in cands],
                 "fill_patch_level0": {"ms": round(fill_ms, 4),
@@ -1114,13 +1118,13 @@ def main():
     lib, fns = mx.load()
     fields = w.pass_fields()
     tuned = None
-    # the library's defaults
-    shape = {"tile": "16x11", "tz": 32}
+    # the library's defaults (it picks the chunks from the launch's boxes)
+    shape = {"tile": "16x11", "tz": "picked"}
     if args.autotune and not args.no_autotune:
         # the autotuner picks the fused edge kernel's tile and z-chunk on
         # this workload (untimed, before the warm-up)
         cands, best = m.autotune([fields])
-        tuned = {"tile": TILE_NAMES[cands[best][0]], "tz": cands[best][1]}
+        tuned = tuned_shape(cands[best])
         shape = dict(tuned)
         print(f"[bench] autotune {[(c[0], c[1], round(c[2], 3)) for c in cands]} -> {tuned}",
               file=sys.stderr, flush=True)
@@ -1194,8 +1198,10 @@ def main():
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
+        # measured on boxes of 128^3, from which the chunks are picked
         "traffic": committed_traffic(
-            dname, f"{args.n}c_ppm{args.ppm}_{shape['tile']}_tz{shape['tz']}"),
+            dname, f"{args.n}c_ppm{args.ppm}_{shape['tile']}_tz{shape['tz']}")
+        if args.max_grid == 128 and not args.spherical else None,
         "avg_launch_ms": round(avg_ms, 4),
         "bytes_per_cell": bpc,
         "pass_achieved": round(pass_gbs, 2),

@@ -254,12 +254,13 @@ __device__ __forceinline__ double tape_dir(const AB& A, const PT& P, const doubl
 }
 
 //
-// The tape's kernels are bound by the L1 path (its address and data units are
-// busy all the time, some 16 cycles per load and as many again on misses) and by
-// the limiters' FP64 work, so each evaluates a face's upwind cell only and keeps
-// one predictor state per face instead of both sides' and their choice.  128^3 of
-// 4 components, ppm_type 1, against both sides at every face: this kernel 265 ->
-// 150 us, the corner states 350 -> 250 us, the edge states 440 -> 340 us.
+// The tape's kernels are bound by the L1 path (128^3 of 4 components, ppm_type 1: its
+// address unit is busy 70 to 94% of the cycles and its data unit 91 to 96%, with 17
+// accesses per instruction), by HBM (4.1 to 4.7 TB/s of the 5.0 of a copy) and, this
+// one, by the limiters' FP64 work (VALU issue 80%).  So each evaluates a face's upwind
+// cell only and keeps one predictor state per face instead of both sides' and their
+// choice; against both sides at every face: this kernel 265 -> 150 us, the corner
+// states 350 -> 250 us, the edge states 440 -> 340 us.
 template <int PPM, class PT>
 __global__ void __launch_bounds__(NTB) k_tape_ppm(AB A) {
     const PT P = PT::make(A);

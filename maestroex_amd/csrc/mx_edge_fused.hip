@@ -40,13 +40,15 @@
 // paths are predicated.
 //
 // What bounds it: VALU issue and the latency of the dependent FP64 chains
-// between barriers, not HBM (3.5 + 2.6 GB move per 256^3 launch of 5 scalars).
+// between barriers, then HBM.  A 256^3 launch of 5 scalars (ppm_type 1, 2.73 ms)
+// issues VALU for 1.66 ms (56 to 61%), its waves wait for half of their cycles,
+// and 9.8 GB move (7.2 read, 2.6 written), 3.6 TB/s, 70% of what a copy reaches.
 // One wave alone takes 10.7 thousand cycles a step for 510 VALU instructions,
 // so waves in flight decide: the advective ppm_type 1 kernel is held to 128
 // VGPRs and 40 KB of LDS, 4 blocks a CU (3.11 ms at 3 blocks, 2.68 ms at 4).
 // Measured per 256^3 launch against evaluating both sides of every face in
-// seven phases: ppm_type 1 2.68 ms (3.74), VALU 65% busy (55%); ppm_type 2
-// 4.51 ms (5.48); conservative, 128^3 and 3 species, 0.38 ms (0.46).
+// seven phases: ppm_type 1 2.68 ms (3.74); ppm_type 2 4.51 ms (5.48);
+// conservative, 128^3 and 3 species, 0.38 ms (0.46).
 #include <algorithm>
 #include <climits>
 

@@ -139,9 +139,13 @@ struct mx_adv_ctx {
     int adj_face_sums = 0;    // adjoint: predictor-state face adjoints stored once per face
     int adj_pow2 = 1;         // adjoint: mask indexing when n is a power of two
     int adj_trace_rolled = 0; // adjoint: trace kernel with one direction per loop trip
-    int adj_xcd = -1;         // adjoint: each XCD takes a contiguous range of blocks; -1: over
-                              // box lists (90 x 75 x 110 of 2 components, ppm_type 2: 844 -> 801
-                              // us), not on one periodic box (128^3 of 4: 2478 against 2494 us)
+    // adjoint: each XCD takes a contiguous range of blocks; -1: over box lists, not on
+    // one periodic box.  Step and gradient, on against off, 1 to 4 components, ppm_type
+    // 1 and 2: box lists of 24^3 to 130 x 30 x 60 and 90 x 75 x 110 (2 components,
+    // ppm_type 2: 799 -> 767 us) 0.90 to 1.00, of 64^3 and 128^3, whose strides are
+    // powers of two, 0.96 to 1.02; periodic boxes 0.88 (97^3 of 1) to 1.00 up to 129^3,
+    // but 1.01 to 1.02 on 128^3 of 4, for which it is off, and 1.00 to 1.01 on 136^3
+    int adj_xcd = -1;
 
     // calls that allocate nothing (mx_adv_advance_pass_noalloc).  With `dry`
     // set an entry point runs its host logic only: every launch is skipped,

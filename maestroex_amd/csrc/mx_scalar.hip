@@ -1110,11 +1110,13 @@ int advance_pass_levels(mx_adv_ctx* c, int lev0, int nlev, const mx_adv_pass_arg
             for (int n = 0; n < gr[1]; ++n) sc.push_back(gr[0] + n);
         if ((rc = make_edge_scal_fused_list(c, levs, 0, bs, sc, sc, 0))) return rc;
     } else {
-        // the staged kernels take the three calls in one, too, where the calls'
-        // own launches count (four of the 16 of a 2-D pass, 256^2: 103 -> 88 us)
-        // and the temporaries of all their components at once are small (half of
-        // the allocation-free pass's scratch, whose sizing run and whose run must
-        // choose alike)
+        // the staged kernels take the three calls in one, too: four launches fewer.
+        // The temporaries are then of all their components at once, so up to half
+        // of the allocation-free pass's scratch only (whose sizing run and whose run
+        // must choose alike).  The pass, one call against three: 256^2 95 -> 76 us,
+        // 48^3 with ppm_type 0 (57 MiB) 256 -> 227, 768^2 (90 MiB) 272 -> 259;
+        // above the line 1024^2 (161 MiB) would take 0.97 of the time, 2048^2 (641
+        // MiB) 1.00
         std::vector<int> all;
         for (const auto& gr : groups)
             for (int n = 0; n < gr[1]; ++n) all.push_back(gr[0] + n);

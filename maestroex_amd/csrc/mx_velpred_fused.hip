@@ -4,7 +4,12 @@
 // (MaestroVelPred.cpp:5-292 with VelPredInterface :735-1128,
 // VelPredTransverse :1130-1595 and VelPredVelocities :1597-1915).
 //
-// A block owns a TX x TY tile of cell columns of one box, grown by one cell
+// Two kernels.  k_vp_fused_comp, the one in use: one velocity component per block,
+// upwind first, three phases a plane (described above its code).  k_vp_fused: all
+// three components per block, both sides of every face, for FABs whose rows the
+// other's 32-bit offsets do not reach, and as the choice "velpred_fused_comp" 0.
+//
+// In both a block owns a TX x TY tile of cell columns of one box, grown by one cell
 // in x and y (one thread per column), and marches up a chunk [z0, z1] of the
 // box's planes, one cell plane q per step (plus q = z0 - 1 and q = z1 + 1).
 // Nothing goes through HBM between the stages: the reference's sixteen
@@ -20,15 +25,15 @@
 //
 // The reference formulas are regrouped, not changed: a transverse correction
 // (dt/6h_T)(utrans_T(+) + utrans_T(-))(uimh_T(+) - uimh_T(-)) depends only on
-// the cell it is taken across, so it is evaluated once per cell and read by
-// the faces on both sides; the final corrections (dt/4h_T) likewise.  Each is
+// the cell it is taken across; the final corrections (dt/4h_T) likewise.  Each is
 // the reference's expression in the reference's operand order, so the
 // results are bit-identical to the per-point kernels.  PPM boundary stencils
 // (ext_dir / hoextrap within three cells of a domain side) use the full
 // per-cell routine of mx_device.H; the tracing velocity is ufull at the cell
 // (is_umac = 0).
 //
-// Per step q, phases separated by barriers:
+// k_vp_fused evaluates a correction once per cell for the faces on both sides.  Per
+// step q, phases separated by barriers:
 //   A  stage plane q of the three components and of utrans_x, utrans_y;
 //      shift the column's z windows; issue the loads of plane q + 1;
 //   B1 face values of plane q (x, y, three components); PPM of cell q in z
