@@ -925,10 +925,15 @@ int launch_fused(mx_adv_ctx* c, const std::vector<EdgeLevel>& levs, int tz, int 
         }
     }
     if (tz <= 0) {
-        // of the two launches' kernels
-        const int blocks[2] = {zgen ? fused_blocks<TX, TY, 1>(c->p.ppm_type, cons)
-                                    : fused_blocks<TX, TY, 0>(c->p.ppm_type, cons),
-                               fused_blocks<TX, TY, 2>(c->p.ppm_type, cons)};
+        // of the kernels that the launches take (a query loads its kernel)
+        bool any[2] = {false, false};
+        for (const ChunkCols& col : cols)
+            for (int l = 0; l < 2; ++l) any[l] = any[l] || col.tiles[l];
+        const int ppm = c->p.ppm_type;
+        const int blocks[2] = {!any[0] ? 1
+                               : zgen  ? fused_blocks<TX, TY, 1>(ppm, cons)
+                                       : fused_blocks<TX, TY, 0>(ppm, cons),
+                               any[1] ? fused_blocks<TX, TY, 2>(ppm, cons) : 1};
         tz = pick_chunks(cols, num_comp, blocks);
     }
     for (size_t id = 0; id < boxes.size(); ++id) {

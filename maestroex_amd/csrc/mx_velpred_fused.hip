@@ -1610,10 +1610,15 @@ int vp_launch(mx_adv_ctx* c, const std::vector<VFBox>& boxes, int tz, bool one_l
             zgen = zgen || (col.tiles[0] && !vf_tile_free(B.lo[2], col.nz, B.domlo[2], B.domhi[2],
                                                           act[2][0], act[2][1]));
         }
-        // of the two launches' kernels
+        // of the kernels that the launches take (a query loads its kernel)
+        bool any[2] = {false, false};
+        for (const ChunkCols& col : cols)
+            for (int l = 0; l < 2; ++l) any[l] = any[l] || col.tiles[l];
         const int ppm = c->p.ppm_type;
-        const int blocks[2] = {zgen ? vp_blocks<TX, TY, 1, WPE>(ppm) : vp_blocks<TX, TY, 0, WPE>(ppm),
-                               vp_blocks<TX, TY, 2, WPE>(ppm)};
+        const int blocks[2] = {!any[0] ? 1
+                               : zgen  ? vp_blocks<TX, TY, 1, WPE>(ppm)
+                                       : vp_blocks<TX, TY, 0, WPE>(ppm),
+                               any[1] ? vp_blocks<TX, TY, 2, WPE>(ppm) : 1};
         tz = pick_chunks(cols, 3, blocks);
     }
     std::vector<VPTile> tiles, btiles;  // clear of general x/y sides, the others
